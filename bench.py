@@ -506,7 +506,9 @@ def main():
         # algorithmic bytes per complex point of one launch (one read + one write of the transform's input and
         # output, intermediates not counted): 16 for a single-pass kernel, 8 for each pass of the four-step (the
         # column pass reads the input, the row pass writes the output; the intermediate between them is excluded)
-        two_pass = info["algorithm"] == 2
+        two_pass = info["algorithm"] == 2 and acc.launches[1] > 0
+        if info["algorithm"] == 2 and not two_pass:
+            names[0] = "whole transforms (both four-step passes on one CU each)"
         kernels = []
         for ph in range(4):
             if acc.launches[ph] == 0:

@@ -100,6 +100,24 @@ struct FusedArgs
     uint32_t hints;
 };
 
+// Whole transforms of n = 256 * n2 = 2^15 or 2^16 points, one per workgroup of a persistent launch (k_whole).
+struct WholeArgs
+{
+    const cfloat* in;
+    cfloat* out;
+    const cfloat* roots; // W_256^e, e < 256
+    const cfloat* tfull; // W_n^{c k1} at [c * 256 + k1]
+    uint64_t count;
+    uint64_t idist;
+    uint64_t odist;
+    float scale;
+    uint32_t stagger = 0; // set by the launcher
+};
+// Whether k_whole runs n, and the n2 its twiddle table is laid out for.
+bool whole_kernel_n(uint64_t n, uint64_t* n2);
+// grid: workgroups at most (one per CU).
+hipError_t launch_whole(uint64_t n, bool inverse, const WholeArgs& a, unsigned grid, hipStream_t s);
+
 // One square transform n = n1 * n1 split over a group of workgroups of one XCD (k_coop): each member runs one
 // column tile and one row tile of every transform its group takes, and the group's n-point slot is shared through
 // that XCD's L2. Groups form at launch from the XCC_ID each workgroup reads; a launch that does not become resident

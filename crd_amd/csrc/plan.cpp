@@ -138,6 +138,11 @@ struct crdfft_plan_s
     DeviceBuffer thi, tlo;  // factored four-step twiddle
     DeviceBuffer tstep;     // column pass step table (e1 * n2 entries)
     DeviceBuffer tfull;     // column pass full twiddle table (n entries, small n only)
+    // whole-transform kernel of n = 2^15, 2^16 C2C (untuned plans): W_256^e and the full four-step twiddle of
+    // 256 x n / 256; whole_cus > 0 when the plan has it
+    DeviceBuffer whole_roots, whole_full;
+    uint32_t whole_cus = 0;
+    bool whole_always = false; // the self-check's plan of one transform: whatever the batch
     uint32_t hshift = 0;
     DeviceBuffer wreal;     // W_n^k, k <= n/2, for R2C/C2R
     DeviceBuffer wref;      // W_cn^k, k < cn/2, for the radix-2 reference (built on first use)
@@ -248,6 +253,21 @@ struct Profiler
         return err;
     }
 };
+
+crdfft_status build_whole_tables(crdfft_plan_s* p, hipStream_t s)
+{
+    const uint64_t cn = p->shape.complex_n;
+    uint64_t n2 = 0;
+    if (!crdfft::whole_kernel_n(cn, &n2))
+    {
+        return CRDFFT_UNSUPPORTED;
+    }
+    CRDFFT_TRY(p->whole_roots.alloc(256 * sizeof(cfloat)));
+    CRDFFT_TRY(crdfft::build_roots(p->whole_roots.as<cfloat>(), 256, 1, 256, s));
+    CRDFFT_TRY(p->whole_full.alloc(cn * sizeof(cfloat)));
+    CRDFFT_TRY(crdfft::build_full_twiddle(p->whole_full.as<cfloat>(), n2, 256, cn, s));
+    return CRDFFT_OK;
+}
 
 crdfft_status build_tables(crdfft_plan_s* p, hipStream_t s)
 {
@@ -387,6 +407,14 @@ crdfft_status build_tables(crdfft_plan_s* p, hipStream_t s)
         }
         CRDFFT_TRY(p->workspace.alloc(sh.workspace_bytes));
     }
+    if (p->whole_cus > 0)
+    {
+        const crdfft_status st = build_whole_tables(p, s);
+        if (st != CRDFFT_OK)
+        {
+            return st;
+        }
+    }
     if (sh.type != CRDFFT_C2C)
     {
         const uint64_t h = sh.n / 2;
@@ -394,6 +422,21 @@ crdfft_status build_tables(crdfft_plan_s* p, hipStream_t s)
         CRDFFT_TRY(crdfft::build_roots(p->wreal.as<cfloat>(), h + 1, 1, sh.n, s));
     }
     return CRDFFT_OK;
+}
+
+// Of `count` transforms, how many the whole-transform kernel runs (the first ones; the four-step runs the rest). It takes
+// rounds of one transform per CU, so a partial round costs nearly a full one (256 CUs, n = 2^16 / 2^15: 60 / 26 us with
+// 96 transforms, 73 / 32 with 256) and the four-step about 0.37 / 0.21 us per transform. Alone, a partial round pays from
+// 176 / 128 transforms on (whole 66 / 27 us, four-step 67 / 28); behind full rounds it overlaps them and pays sooner: from
+// 96 (352 transforms: whole 126 / 60 us, split 126 / 64; 576, a rest of 64: 189 / 94, split 180 / 88), and behind four of
+// them from about 32 (1088, a rest of 64: 300 / 140, split 309 / 148).
+uint64_t whole_count(const crdfft_plan_s* p, uint64_t count)
+{
+    const uint64_t cus = p->whole_cus;
+    const uint64_t full = count / cus, rest = count % cus;
+    const uint64_t least = full == 0 ? (p->shape.complex_n == 65536 ? cus * 11 / 16 : cus / 2)
+                                     : (full < 4 ? cus * 3 / 8 : cus / 8);
+    return p->whole_always || rest >= least ? count : count - rest;
 }
 
 // The complex transform of the plan over `count` transforms (complex distances), on `s`.
@@ -439,6 +482,29 @@ crdfft_status run_complex(crdfft_plan_s* p, const cfloat* in, cfloat* out, uint6
         }
         case CRDFFT_ALGO_FOUR_STEP:
         {
+            // in place only where a transform's input and output are the same points: each workgroup reads its next
+            // transform before it has written the current one
+            if (p->whole_cus > 0 && r2c_w == nullptr && c2r_w == nullptr &&
+                (in == out ? idist == odist || count == 1
+                           : in + (count - 1) * idist + cn <= out || out + (count - 1) * odist + cn <= in))
+            {
+                const uint64_t whole = whole_count(p, count);
+                if (whole > 0)
+                {
+                    const crdfft::WholeArgs wa{in, out, p->whole_roots.as<cfloat>(), p->whole_full.as<cfloat>(),
+                                               whole, idist, odist, scale};
+                    CRDFFT_TRY(prof.before());
+                    CRDFFT_TRY(crdfft::launch_whole(cn, inverse, wa, p->whole_cus, s));
+                    CRDFFT_TRY(prof.after(0, cn * whole));
+                    in += whole * idist;
+                    out += whole * odist;
+                    count -= whole;
+                }
+                if (count == 0)
+                {
+                    return CRDFFT_OK;
+                }
+            }
             const crdfft::ScratchOverride* ov = crdfft::scratch_override();
             uint64_t chunk = sh.chunk;
             cfloat* ws = nullptr;
@@ -870,6 +936,16 @@ crdfft_status create_plan(crdfft_plan* plan, uint64_t n, uint64_t batch, uint64_
     p->odist = odist;
     p->flags = flags;
     (void)hipGetDevice(&p->device);
+    uint64_t whole_n2 = 0;
+    if (tuning == nullptr && type == CRDFFT_C2C && shape.algorithm == CRDFFT_ALGO_FOUR_STEP &&
+        precision == CRDFFT_FP32 && crdfft::whole_kernel_n(shape.complex_n, &whole_n2))
+    {
+        int cus = 0;
+        if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, p->device) == hipSuccess && cus > 0)
+        {
+            p->whole_cus = static_cast<uint32_t>(cus);
+        }
+    }
     crdfft_status rs = build_tables(p, nullptr);
     if (rs == CRDFFT_OK)
     {
@@ -1149,6 +1225,21 @@ crdfft_status plan_use_floor(crdfft_plan p)
     }
     p->floor = true;
     return CRDFFT_OK;
+}
+
+bool plan_uses_whole(crdfft_plan p) { return p->whole_cus > 0 && whole_count(p, p->shape.batch) > 0; }
+
+bool plan_uses_four_step(crdfft_plan p)
+{
+    // (different distances: an in-place execute, which the whole-transform kernel cannot run)
+    return p->whole_cus == 0 || p->idist != p->odist || whole_count(p, p->shape.batch) < p->shape.batch;
+}
+
+crdfft_status plan_use_whole(crdfft_plan p)
+{
+    p->whole_cus = 1;
+    p->whole_always = true;
+    return build_whole_tables(p, nullptr);
 }
 
 bool plan_on_floor(crdfft_plan p) { return p != nullptr && p->floor; }

@@ -141,8 +141,20 @@ extern "C" crdfft_status crdfft_self_check(crdfft_plan plan)
             return st;
         }
         crdfft_status result = CRDFFT_OK;
-        for (int dir = 0; dir < 2 && result == CRDFFT_OK; ++dir)
+        // both directions on the four-step or single kernel, then on the whole-transform kernel, as the plan uses them
+        const bool whole = !crdfft::plan_on_floor(plan) && crdfft::plan_uses_whole(plan);
+        const int first = whole && !crdfft::plan_uses_four_step(plan) ? 2 : 0;
+        for (int form = first; form < (whole ? 4 : 2) && result == CRDFFT_OK; ++form)
         {
+            const int dir = form & 1;
+            if (form == 2)
+            {
+                result = crdfft::plan_use_whole(one);
+                if (result != CRDFFT_OK)
+                {
+                    break;
+                }
+            }
             for (uint64_t c = 0; c < cases && result == CRDFFT_OK; ++c)
             {
                 for (uint64_t j = 0; j < n; ++j)
