@@ -112,11 +112,15 @@ struct WholeArgs
     uint64_t odist;
     float scale;
     uint32_t stagger = 0; // set by the launcher
+    const cfloat* wreal = nullptr; // launch_whole_real: W_2h^k, k <= h
 };
 // Whether k_whole runs n, and the n2 its twiddle table is laid out for.
 bool whole_kernel_n(uint64_t n, uint64_t* n2);
 // grid: workgroups at most (one per CU).
 hipError_t launch_whole(uint64_t n, bool inverse, const WholeArgs& a, unsigned grid, hipStream_t s);
+// The real transforms of 2h = 2^16 reals on the same kernel (h = 2^15): R2C from h pairs to h + 1 bins, C2R back (scaled
+// 1 / 2h); distances in complex elements.
+hipError_t launch_whole_real(uint64_t h, bool c2r, const WholeArgs& a, unsigned grid, hipStream_t s);
 
 // One square transform n = n1 * n1 split over a group of workgroups of one XCD (k_coop): each member runs one
 // column tile and one row tile of every transform its group takes, and the group's n-point slot is shared through

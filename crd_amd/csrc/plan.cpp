@@ -138,8 +138,8 @@ struct crdfft_plan_s
     DeviceBuffer thi, tlo;  // factored four-step twiddle
     DeviceBuffer tstep;     // column pass step table (e1 * n2 entries)
     DeviceBuffer tfull;     // column pass full twiddle table (n entries, small n only)
-    // whole-transform kernel of n = 2^15, 2^16 C2C (untuned plans): W_256^e and the full four-step twiddle of
-    // 256 x n / 256; whole_cus > 0 when the plan has it
+    // whole-transform kernel of n = 2^15, 2^16 C2C and n = 2^16 R2C / C2R (untuned plans): W_256^e and the full
+    // four-step twiddle of 256 x complex_n / 256; whole_cus > 0 when the plan has it
     DeviceBuffer whole_roots, whole_full;
     uint32_t whole_cus = 0;
     bool whole_always = false; // the self-check's plan of one transform: whatever the batch
@@ -484,7 +484,7 @@ crdfft_status run_complex(crdfft_plan_s* p, const cfloat* in, cfloat* out, uint6
         {
             // in place only where a transform's input and output are the same points: each workgroup reads its next
             // transform before it has written the current one
-            if (p->whole_cus > 0 && r2c_w == nullptr && c2r_w == nullptr &&
+            if (p->whole_cus > 0 && sh.type == CRDFFT_C2C &&
                 (in == out ? idist == odist || count == 1
                            : in + (count - 1) * idist + cn <= out || out + (count - 1) * odist + cn <= in))
             {
@@ -673,6 +673,32 @@ crdfft_status run_complex(crdfft_plan_s* p, const cfloat* in, cfloat* out, uint6
     }
 }
 
+// The first transforms of an R2C or C2R plan of n = 2^16 on the whole-transform kernel (distances in complex elements);
+// *whole = how many (0 where the plan has no such kernel, or where input and output overlap).
+crdfft_status run_whole_real(crdfft_plan_s* p, const cfloat* in, cfloat* out, uint64_t idist, uint64_t odist,
+                             hipStream_t s, Profiler& prof, uint64_t* whole)
+{
+    const crdfft::PlanShape& sh = p->shape;
+    const bool c2r = sh.type == CRDFFT_C2R;
+    const uint64_t in_len = sh.complex_n + (c2r ? 1 : 0), out_len = sh.complex_n + (c2r ? 0 : 1);
+    *whole = 0;
+    if (p->whole_cus == 0 || p->floor ||
+        !(in + (sh.batch - 1) * idist + in_len <= out || out + (sh.batch - 1) * odist + out_len <= in))
+    {
+        return CRDFFT_OK;
+    }
+    *whole = whole_count(p, sh.batch);
+    if (*whole > 0)
+    {
+        crdfft::WholeArgs wa{in, out, p->whole_roots.as<cfloat>(), p->whole_full.as<cfloat>(), *whole, idist, odist, 1.0f};
+        wa.wreal = p->wreal.as<cfloat>();
+        CRDFFT_TRY(prof.before());
+        CRDFFT_TRY(crdfft::launch_whole_real(sh.complex_n, c2r, wa, p->whole_cus, s));
+        CRDFFT_TRY(prof.after(0, sh.complex_n * *whole));
+    }
+    return CRDFFT_OK;
+}
+
 crdfft_status execute_impl(crdfft_plan p, const void* in, void* out, int32_t direction, void* stream, Profiler& prof)
 {
     if (p == nullptr || in == nullptr || out == nullptr ||
@@ -828,13 +854,20 @@ crdfft_status execute_impl(crdfft_plan p, const void* in, void* out, int32_t dir
                 CRDFFT_TRY(prof.after(0, h * sh.batch));
                 return CRDFFT_OK;
             }
+            uint64_t whole = 0;
+            crdfft_status wst = run_whole_real(p, static_cast<const cfloat*>(in), o, p->idist / 2, p->odist, s, prof, &whole);
+            if (wst != CRDFFT_OK || whole == sh.batch)
+            {
+                return wst;
+            }
             if (sh.algorithm == CRDFFT_ALGO_FOUR_STEP && (p->flags & CRDFFT_FLAG_SEPARATE_PASSES) == 0 && !p->floor &&
                 (sh.hints & crdfft::kHintPersistent) == 0 && crdfft::have_rowtr_r2c(sh.n2, sh.e2, sh.tile2) &&
                 sh.n1 >= static_cast<uint64_t>(sh.tile2))
             {
                 // n > 32768: the column pass, then the row pass with the recombine fused in (two passes, not three)
-                return run_complex(p, static_cast<const cfloat*>(in), o, sh.batch, p->idist / 2, p->odist, false, s,
-                                   prof, 1.0f, p->wreal.as<cfloat>());
+                return run_complex(p, static_cast<const cfloat*>(in) + whole * (p->idist / 2), o + whole * p->odist,
+                                   sh.batch - whole, p->idist / 2, p->odist, false, s, prof, 1.0f,
+                                   p->wreal.as<cfloat>());
             }
             const crdfft_status st =
                 run_complex(p, static_cast<const cfloat*>(in), o, sh.batch, p->idist / 2, p->odist, false, s, prof);
@@ -869,13 +902,20 @@ crdfft_status execute_impl(crdfft_plan p, const void* in, void* out, int32_t dir
                 CRDFFT_TRY(prof.after(0, h * sh.batch));
                 return CRDFFT_OK;
             }
+            uint64_t whole = 0;
+            crdfft_status wst = run_whole_real(p, static_cast<const cfloat*>(in), o, p->idist, p->odist / 2, s, prof, &whole);
+            if (wst != CRDFFT_OK || whole == sh.batch)
+            {
+                return wst;
+            }
             if (sh.algorithm == CRDFFT_ALGO_FOUR_STEP && (p->flags & CRDFFT_FLAG_SEPARATE_PASSES) == 0 && !p->floor &&
                 (sh.hints & crdfft::kHintPersistent) == 0 && crdfft::have_cols_c2r(sh.n1, sh.e1, sh.tile1) &&
                 sh.n2 % static_cast<uint64_t>(sh.tile1) == 0)
             {
                 // n > 32768: the pre-rotation in the column pass's loads, then the inverse row pass (two passes)
-                return run_complex(p, static_cast<const cfloat*>(in), o, sh.batch, p->idist, p->odist / 2, true, s,
-                                   prof, 1.0f, nullptr, p->wreal.as<cfloat>());
+                return run_complex(p, static_cast<const cfloat*>(in) + whole * p->idist, o + whole * (p->odist / 2),
+                                   sh.batch - whole, p->idist, p->odist / 2, true, s, prof, 1.0f, nullptr,
+                                   p->wreal.as<cfloat>());
             }
             CRDFFT_TRY(prof.before());
             CRDFFT_TRY(crdfft::launch_c2r_pre(static_cast<const cfloat*>(in), o, p->wreal.as<cfloat>(), h, sh.batch,
@@ -937,8 +977,9 @@ crdfft_status create_plan(crdfft_plan* plan, uint64_t n, uint64_t batch, uint64_
     p->flags = flags;
     (void)hipGetDevice(&p->device);
     uint64_t whole_n2 = 0;
-    if (tuning == nullptr && type == CRDFFT_C2C && shape.algorithm == CRDFFT_ALGO_FOUR_STEP &&
-        precision == CRDFFT_FP32 && crdfft::whole_kernel_n(shape.complex_n, &whole_n2))
+    if (tuning == nullptr && shape.algorithm == CRDFFT_ALGO_FOUR_STEP && precision == CRDFFT_FP32 &&
+        crdfft::whole_kernel_n(shape.complex_n, &whole_n2) &&
+        (type == CRDFFT_C2C || (shape.complex_n == 32768 && (flags & CRDFFT_FLAG_SEPARATE_PASSES) == 0)))
     {
         int cus = 0;
         if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, p->device) == hipSuccess && cus > 0)
@@ -1232,7 +1273,8 @@ bool plan_uses_whole(crdfft_plan p) { return p->whole_cus > 0 && whole_count(p, 
 bool plan_uses_four_step(crdfft_plan p)
 {
     // (different distances: an in-place execute, which the whole-transform kernel cannot run)
-    return p->whole_cus == 0 || p->idist != p->odist || whole_count(p, p->shape.batch) < p->shape.batch;
+    return p->whole_cus == 0 || (p->shape.type == CRDFFT_C2C && p->idist != p->odist) ||
+           whole_count(p, p->shape.batch) < p->shape.batch;
 }
 
 crdfft_status plan_use_whole(crdfft_plan p)

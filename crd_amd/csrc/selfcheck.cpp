@@ -251,92 +251,106 @@ extern "C" crdfft_status crdfft_self_check(crdfft_plan plan)
         return st;
     }
     crdfft_status result = CRDFFT_OK;
-    if (info.type == CRDFFT_R2C)
+    // on the four-step or single kernel, then on the whole-transform kernel, as the plan uses them
+    const bool whole = !crdfft::plan_on_floor(plan) && crdfft::plan_uses_whole(plan);
+    const int first = whole && !crdfft::plan_uses_four_step(plan) ? 1 : 0;
+    for (int form = first; form < (whole ? 2 : 1) && result == CRDFFT_OK; ++form)
     {
-        std::vector<float> x(n);
-        for (uint64_t j = 0; j < n; ++j)
+        if (form == 1)
         {
-            x[j] = static_cast<float>(std::cos(kTwoPi * static_cast<double>(j) / static_cast<double>(n)));
-        }
-        std::vector<std::complex<float>> X(h + 1);
-        if (hipMemcpy(dr.p, x.data(), n * 4, hipMemcpyHostToDevice) != hipSuccess)
-        {
-            result = CRDFFT_HIP_ERROR;
-        }
-        if (result == CRDFFT_OK)
-        {
-            result = crdfft_execute(one, dr.p, dc.p, CRDFFT_FORWARD, nullptr);
-        }
-        if (result == CRDFFT_OK && hipMemcpy(X.data(), dc.p, (h + 1) * 8, hipMemcpyDeviceToHost) != hipSuccess)
-        {
-            result = CRDFFT_HIP_ERROR;
-        }
-        if (result == CRDFFT_OK)
-        {
-            if (fault)
+            result = crdfft::plan_use_whole(one);
+            if (result != CRDFFT_OK)
             {
-                X[1] = std::complex<float>(X[1].real() * 1.5f, X[1].imag());
-            }
-            double maxerr = 0.0;
-            for (uint64_t k = 0; k <= h; ++k)
-            {
-                if (!checked(k, h + 1))
-                {
-                    continue;
-                }
-                const double want = (k == 1) ? static_cast<double>(h) : 0.0;
-                const double err = std::abs(std::complex<double>(X[k].real() - want, X[k].imag()));
-                if (!(err <= maxerr))
-                {
-                    maxerr = err;
-                }
-            }
-            if (!(maxerr <= tol * (1.0 + static_cast<double>(h))))
-            {
-                result = CRDFFT_SELF_CHECK_FAILED;
+                break;
             }
         }
-    }
-    else
-    {
-        std::vector<std::complex<float>> X(h + 1, std::complex<float>(0.0f, 0.0f));
-        X[1] = std::complex<float>(static_cast<float>(h), 0.0f);
-        std::vector<float> x(n);
-        if (hipMemcpy(dc.p, X.data(), (h + 1) * 8, hipMemcpyHostToDevice) != hipSuccess)
+        if (info.type == CRDFFT_R2C)
         {
-            result = CRDFFT_HIP_ERROR;
-        }
-        if (result == CRDFFT_OK)
-        {
-            result = crdfft_execute(one, dc.p, dr.p, CRDFFT_INVERSE, nullptr);
-        }
-        if (result == CRDFFT_OK && hipMemcpy(x.data(), dr.p, n * 4, hipMemcpyDeviceToHost) != hipSuccess)
-        {
-            result = CRDFFT_HIP_ERROR;
-        }
-        if (result == CRDFFT_OK)
-        {
-            if (fault)
-            {
-                x[0] += 0.5f;
-            }
-            double maxerr = 0.0;
+            std::vector<float> x(n);
             for (uint64_t j = 0; j < n; ++j)
             {
-                if (!checked(j, n))
+                x[j] = static_cast<float>(std::cos(kTwoPi * static_cast<double>(j) / static_cast<double>(n)));
+            }
+            std::vector<std::complex<float>> X(h + 1);
+            if (hipMemcpy(dr.p, x.data(), n * 4, hipMemcpyHostToDevice) != hipSuccess)
+            {
+                result = CRDFFT_HIP_ERROR;
+            }
+            if (result == CRDFFT_OK)
+            {
+                result = crdfft_execute(one, dr.p, dc.p, CRDFFT_FORWARD, nullptr);
+            }
+            if (result == CRDFFT_OK && hipMemcpy(X.data(), dc.p, (h + 1) * 8, hipMemcpyDeviceToHost) != hipSuccess)
+            {
+                result = CRDFFT_HIP_ERROR;
+            }
+            if (result == CRDFFT_OK)
+            {
+                if (fault)
                 {
-                    continue;
+                    X[1] = std::complex<float>(X[1].real() * 1.5f, X[1].imag());
                 }
-                const double want = std::cos(kTwoPi * static_cast<double>(j) / static_cast<double>(n));
-                const double err = std::abs(static_cast<double>(x[j]) - want);
-                if (!(err <= maxerr))
+                double maxerr = 0.0;
+                for (uint64_t k = 0; k <= h; ++k)
                 {
-                    maxerr = err;
+                    if (!checked(k, h + 1))
+                    {
+                        continue;
+                    }
+                    const double want = (k == 1) ? static_cast<double>(h) : 0.0;
+                    const double err = std::abs(std::complex<double>(X[k].real() - want, X[k].imag()));
+                    if (!(err <= maxerr))
+                    {
+                        maxerr = err;
+                    }
+                }
+                if (!(maxerr <= tol * (1.0 + static_cast<double>(h))))
+                {
+                    result = CRDFFT_SELF_CHECK_FAILED;
                 }
             }
-            if (!(maxerr <= tol * 2.0))
+        }
+        else
+        {
+            std::vector<std::complex<float>> X(h + 1, std::complex<float>(0.0f, 0.0f));
+            X[1] = std::complex<float>(static_cast<float>(h), 0.0f);
+            std::vector<float> x(n);
+            if (hipMemcpy(dc.p, X.data(), (h + 1) * 8, hipMemcpyHostToDevice) != hipSuccess)
             {
-                result = CRDFFT_SELF_CHECK_FAILED;
+                result = CRDFFT_HIP_ERROR;
+            }
+            if (result == CRDFFT_OK)
+            {
+                result = crdfft_execute(one, dc.p, dr.p, CRDFFT_INVERSE, nullptr);
+            }
+            if (result == CRDFFT_OK && hipMemcpy(x.data(), dr.p, n * 4, hipMemcpyDeviceToHost) != hipSuccess)
+            {
+                result = CRDFFT_HIP_ERROR;
+            }
+            if (result == CRDFFT_OK)
+            {
+                if (fault)
+                {
+                    x[0] += 0.5f;
+                }
+                double maxerr = 0.0;
+                for (uint64_t j = 0; j < n; ++j)
+                {
+                    if (!checked(j, n))
+                    {
+                        continue;
+                    }
+                    const double want = std::cos(kTwoPi * static_cast<double>(j) / static_cast<double>(n));
+                    const double err = std::abs(static_cast<double>(x[j]) - want);
+                    if (!(err <= maxerr))
+                    {
+                        maxerr = err;
+                    }
+                }
+                if (!(maxerr <= tol * 2.0))
+                {
+                    result = CRDFFT_SELF_CHECK_FAILED;
+                }
             }
         }
     }

@@ -1,4 +1,4 @@
-"""The whole-transform kernel of n = 2^15 and 2^16 C2C (one workgroup per transform, persistent over rounds of one
+"""The whole-transform kernel of n = 2^15 and 2^16 C2C and n = 2^16 R2C / C2R (one workgroup per transform, persistent over rounds of one
 transform per CU) at the batches where its dispatch changes: the smallest partial round it takes, full rounds, a partial
 round behind full ones, and a rest that the four-step runs. Rows of every round against FP64 (rel-L2 <= 2e-6 log2 n), all
 rows against a tuned four-step plan (both within that bound of FP64, so within twice the bound of each other)."""
@@ -76,3 +76,63 @@ def test_rerun_is_bit_identical(gpu):
     a = _run(gpu, plan, x, n, False, gpu.FORWARD, np.complex64(0))
     b = _run(gpu, plan, x, n, True, gpu.FORWARD, np.complex64(0))
     assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
+# rows of h + 1 bins start at every residue of a 128-byte line; padded rows keep one residue
+@pytest.mark.parametrize("batch,pad", [(128, 0), (257, 0), (259, 7), (352, 15), (1056, 1)])
+def test_real_rounds_match_fp64_and_the_four_step(gpu, po, batch, pad):
+    n = 1 << 16
+    h = n // 2
+    pitch = h + 1 + pad
+    print(f"whole real batch={batch} pad={pad}", flush=True)
+    rng = np.random.default_rng(batch + pad)
+    x = rng.standard_normal((batch, n), dtype=np.float32)
+    guard = np.complex64(complex(-3.25, 7.5))
+    r2c = gpu.FftPlan(n, batch, "r2c", odist=pitch)
+    c2r = gpu.FftPlan(n, batch, "c2r", idist=pitch)
+    xin = gpu.DeviceBuffer.from_array(x)
+    spec = gpu.DeviceBuffer.from_array(np.full((batch, pitch), guard, np.complex64))
+    back = gpu.DeviceBuffer(4 * n * batch)
+    r2c.execute(xin, spec, gpu.FORWARD)
+    c2r.execute(spec, back, gpu.INVERSE)
+    gpu.synchronize()
+    X = spec.download((batch, pitch), np.complex64)
+    rows = sorted({0, 1, 2, 15, 16, 127, batch // 2, 255, 256, batch - 1} & set(range(batch)))
+    assert po.rel_l2(X[rows][:, : h + 1], po.rfft64(x[rows].astype(np.float64))) <= bound(n)
+    assert not np.any(X[:, 0].imag) and not np.any(X[:, h].imag)
+    assert np.array_equal(X[:, h + 1:].view(np.uint32), np.full((batch, pad), guard, np.complex64).view(np.uint32))
+    xb = back.download((batch, n), np.float32)
+    assert po.rel_l2(xb, x.astype(np.float64)) <= 2 * bound(n)
+    # the inverse on a spectrum that is no transform of reals at 0 and h: the four-step's formula, all rows
+    X[:, 0] += 1j
+    X[:, h] -= 2j
+    spec2 = gpu.DeviceBuffer.from_array(X)
+    four_r = gpu.FftPlan(n, batch, "r2c", odist=pitch, tuning={"chunk": r2c.info()["chunk"]})
+    four_c = gpu.FftPlan(n, batch, "c2r", idist=pitch, tuning={"chunk": c2r.info()["chunk"]})
+    other = gpu.DeviceBuffer(4 * n * batch)
+    c2r.execute(spec2, back, gpu.INVERSE)
+    four_c.execute(spec2, other, gpu.INVERSE)
+    four_r.execute(xin, spec, gpu.FORWARD)
+    gpu.synchronize()
+    a, b = back.download((batch, n), np.float32), other.download((batch, n), np.float32)
+    Y = spec.download((batch, pitch), np.complex64)
+    for r in range(batch):
+        assert po.rel_l2(a[r], b[r].astype(np.float64)) <= 2 * bound(n), r
+        if r not in rows:
+            assert po.rel_l2(X[r, 1:h], Y[r, 1:h].astype(np.complex128)) <= 2 * bound(n), r
+
+
+def test_rerun_of_the_real_forms_is_bit_identical(gpu):
+    n, batch = 1 << 16, 300
+    h = n // 2
+    x = np.random.default_rng(6).standard_normal((batch, n), dtype=np.float32)
+    r2c, c2r = gpu.FftPlan(n, batch, "r2c"), gpu.FftPlan(n, batch, "c2r")
+    xin, spec, back = gpu.DeviceBuffer.from_array(x), gpu.DeviceBuffer(8 * (h + 1) * batch), gpu.DeviceBuffer(x.nbytes)
+    out = []
+    for _ in range(2):
+        r2c.execute(xin, spec, gpu.FORWARD)
+        c2r.execute(spec, back, gpu.INVERSE)
+        gpu.synchronize()
+        out.append((spec.download((batch, h + 1), np.complex64), back.download((batch, n), np.float32)))
+    for a, b in zip(*out):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
