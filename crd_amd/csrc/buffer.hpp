@@ -66,4 +66,85 @@ template <int AUX> __device__ __forceinline__ void bst(__amdgpu_buffer_rsrc_t r,
                                           static_cast<int>(soff), AUX);
 }
 
+// Which of the sequences of a workgroup (T threads each) a thread belongs to. From T = 64 on the lanes of a wave share
+// it, and saying so (readfirstlane) keeps every address that depends on it in scalar registers. Without it a buffer
+// resource of the sequence counts as divergent and the compiler makes every access a loop over the resources in the wave
+// (11 instructions an iteration), also where there is only one; below T = 64 such loops really run several times, so there
+// Row takes plain accesses. Measured on 2^25-point (real: 2^26-sample) batches: DCT-II n = 8 882 -> 92 us, n = 128 61 -> 47;
+// chirp-z n = 17 (2^23 points) 173 -> 77, n = 61 81 -> 58; STFT of 2^24 samples, frames of 16 / 64 522 -> 97 / 98 -> 49.
+template <int T> __device__ __forceinline__ int slot_of(int tid)
+{
+    if constexpr (T >= 64)
+    {
+        return __builtin_amdgcn_readfirstlane(tid / T);
+    }
+    else
+    {
+        return tid / T;
+    }
+}
+
+// One sequence of `bytes` bytes at `base` (0: an inactive slot, base then any sequence of the call). Offsets in bytes,
+// voff per lane, soff the same in every lane; elements need 4-byte alignment only.
+//   UNIFORM  the same sequence in every lane of a wave: a buffer resource. Loads outside the range return 0, stores
+//            outside are dropped.
+//   else     several sequences per wave: plain accesses. Stores of inactive slots are dropped, their loads read what is
+//            at base; with CHECK every access is held against the range as above.
+template <bool UNIFORM, bool CHECK = false> struct Row;
+
+template <bool CHECK> struct Row<true, CHECK>
+{
+    __amdgpu_buffer_rsrc_t r;
+    __device__ __forceinline__ Row(const void* base, uint32_t bytes) : r(make_rsrc(base, bytes)) {}
+    __device__ __forceinline__ float ld32(uint32_t voff, uint32_t soff) const { return bld32<0>(r, voff, soff); }
+    __device__ __forceinline__ cf ld64(uint32_t voff, uint32_t soff) const { return bld<0>(r, voff, soff); }
+    __device__ __forceinline__ f4v ld128(uint32_t voff, uint32_t soff) const { return bld128<0>(r, voff, soff); }
+    __device__ __forceinline__ void st32(uint32_t voff, uint32_t soff, float v) const { bst32<0>(r, voff, soff, v); }
+    __device__ __forceinline__ void st64(uint32_t voff, uint32_t soff, cf v) const { bst<0>(r, voff, soff, v); }
+    __device__ __forceinline__ void st128(uint32_t voff, uint32_t soff, f4v v) const { bst128<0>(r, voff, soff, v); }
+};
+
+template <bool CHECK> struct Row<false, CHECK>
+{
+    typedef float f2u __attribute__((ext_vector_type(2), aligned(4)));
+    typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+    const char* p;
+    uint32_t n;
+    __device__ __forceinline__ Row(const void* base, uint32_t bytes) : p(static_cast<const char*>(base)), n(bytes) {}
+    template <class V> __device__ __forceinline__ V get(uint32_t off) const
+    {
+        if constexpr (CHECK)
+        {
+            return off < n ? *reinterpret_cast<const V*>(p + off) : V{};
+        }
+        else
+        {
+            return *reinterpret_cast<const V*>(p + off);
+        }
+    }
+    template <class V> __device__ __forceinline__ void put(uint32_t off, V v) const
+    {
+        if (CHECK ? off < n : n != 0)
+        {
+            *reinterpret_cast<V*>(const_cast<char*>(p) + off) = v;
+        }
+    }
+    __device__ __forceinline__ float ld32(uint32_t voff, uint32_t soff) const { return get<float>(voff + soff); }
+    __device__ __forceinline__ cf ld64(uint32_t voff, uint32_t soff) const
+    {
+        const f2u v = get<f2u>(voff + soff);
+        return cf{v.x, v.y};
+    }
+    __device__ __forceinline__ f4v ld128(uint32_t voff, uint32_t soff) const { return get<f4u>(voff + soff); }
+    __device__ __forceinline__ void st32(uint32_t voff, uint32_t soff, float v) const { put<float>(voff + soff, v); }
+    __device__ __forceinline__ void st64(uint32_t voff, uint32_t soff, cf v) const
+    {
+        f2u w;
+        w.x = v.x;
+        w.y = v.y;
+        put<f2u>(voff + soff, w);
+    }
+    __device__ __forceinline__ void st128(uint32_t voff, uint32_t soff, f4v v) const { put<f4u>(voff + soff, v); }
+};
+
 } // namespace crdfft::dev

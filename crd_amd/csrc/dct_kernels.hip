@@ -50,12 +50,12 @@ __global__ __launch_bounds__((DctCfg<H, E>::threads)) void k_dct_fwd(DctArgs a)
     constexpr int N = 2 * H;
     extern __shared__ float lds[];
     const int tid = threadIdx.x;
-    const int local = tid / C::T;
+    const int local = slot_of<C::T>(tid);
     const int i = tid - local * C::T;
     const uint64_t t = static_cast<uint64_t>(blockIdx.x) * C::M + local;
     const bool active = t < a.count;
     const uint32_t row_bytes = active ? static_cast<uint32_t>(N * sizeof(float)) : 0u;
-    const __amdgpu_buffer_rsrc_t rx = make_rsrc(a.in + (active ? t * a.idist : 0), row_bytes);
+    const Row<(C::T >= 64)> rx(a.in + (active ? t * a.idist : 0), row_bytes);
     const LdsView<1> view{lds + local * C::RS, C::LF};
     cf v[E];
     // x[4j..4j+3] = (w[2j], w[n-1-2j], w[2j+1], w[n-2-2j]) for j < h/2: z[j] = (x0, x2) and z[h-1-j] = (x3, x1),
@@ -63,16 +63,15 @@ __global__ __launch_bounds__((DctCfg<H, E>::threads)) void k_dct_fwd(DctArgs a)
 #pragma unroll
     for (int m = 0; m < E / 2; ++m)
     {
-        const int j = i + C::T * m;
-        const f4v q = bld128<0>(rx, static_cast<uint32_t>(j) * 16u, 0);
+        const f4v q = rx.ld128(static_cast<uint32_t>(i) * 16u, C::T * m * 16u);
         v[m] = cf{q.x, q.z};
-        view.put(H - 1 - j, SINE ? cf{-q.w, -q.y} : cf{q.w, q.y});
+        view.put_at(pad16(C::T - 1 - i), C::T * (E - 1 - m), SINE ? cf{-q.w, -q.y} : cf{q.w, q.y});
     }
     __syncthreads();
 #pragma unroll
     for (int m = E / 2; m < E; ++m)
     {
-        v[m] = view.get(i + C::T * m);
+        v[m] = view.get_at(pad16(i), C::T * m);
     }
     __syncthreads();
     fft_core<H, E, false, 1>(v, i, view, reinterpret_cast<const cf*>(a.tw));
@@ -80,12 +79,12 @@ __global__ __launch_bounds__((DctCfg<H, E>::threads)) void k_dct_fwd(DctArgs a)
 #pragma unroll
     for (int m = 0; m < E; ++m)
     {
-        view.put(i + C::T * m, v[m]);
+        view.put_at(pad16(i), C::T * m, v[m]);
     }
     __syncthreads();
     int i2 = i;
     asm volatile("" : "+v"(i2));
-    const __amdgpu_buffer_rsrc_t ry = make_rsrc(a.out + (active ? t * a.odist : 0), row_bytes);
+    const Row<(C::T >= 64)> ry(a.out + (active ? t * a.odist : 0), row_bytes);
     const __amdgpu_buffer_rsrc_t rc = make_rsrc(a.cs, static_cast<uint32_t>((H + 1) * sizeof(cf)));
     const __amdgpu_buffer_rsrc_t rr = make_rsrc(a.rec, static_cast<uint32_t>(H * sizeof(cf)));
     const cf csh = bld<0>(rc, 0, H * sizeof(cf)); // (cos, sin)(pi / 4)
@@ -94,7 +93,9 @@ __global__ __launch_bounds__((DctCfg<H, E>::threads)) void k_dct_fwd(DctArgs a)
     {
         const int k = i2 + C::T * m;
         const cf z = v[m];
-        const cf zp = conjf2(view.get((H - k) & (H - 1)));
+        // element h - k = (T - i) + T (E - 1 - m) for m > 0
+        const cf zp = conjf2(m > 0 && C::T >= 16 ? view.get_at(pad16(C::T - i2), C::T * (E - 1 - m))
+                                                 : view.get((H - k) & (H - 1)));
         const cf A = cf{z.x + zp.x, z.y + zp.y};
         const cf B = cf{z.x - zp.x, z.y - zp.y};
         const cf rb = cmul(B, bld<0>(rr, static_cast<uint32_t>(k) * 8u, 0));
@@ -119,8 +120,8 @@ __global__ __launch_bounds__((DctCfg<H, E>::threads)) void k_dct_fwd(DctArgs a)
             k2 = k > 0 ? static_cast<uint32_t>(N - 1 - k) : static_cast<uint32_t>(H - 1);
             y2 = k > 0 ? cs.x * w2.x + cs.y * w2.y : csh.y * wh;
         }
-        bst32<0>(ry, k1 * 4u, 0, y1);
-        bst32<0>(ry, k2 * 4u, 0, y2);
+        ry.st32(k1 * 4u, 0, y1);
+        ry.st32(k2 * 4u, 0, y2);
     }
 }
 
@@ -131,19 +132,18 @@ __global__ __launch_bounds__((DctCfg<H, E>::threads)) void k_dct_inv(DctArgs a)
     constexpr int N = 2 * H;
     extern __shared__ float lds[];
     const int tid = threadIdx.x;
-    const int local = tid / C::T;
+    const int local = slot_of<C::T>(tid);
     const int i = tid - local * C::T;
     const uint64_t t = static_cast<uint64_t>(blockIdx.x) * C::M + local;
     const bool active = t < a.count;
     const uint32_t row_bytes = active ? static_cast<uint32_t>(N * sizeof(float)) : 0u;
-    const __amdgpu_buffer_rsrc_t rx = make_rsrc(a.in + (active ? t * a.idist : 0), row_bytes);
+    const Row<(C::T >= 64)> rx(a.in + (active ? t * a.idist : 0), row_bytes);
     const LdsView<1> view{lds + local * C::RS, C::LF};
     // the row as pairs (x[2j], x[2j+1]) in the slot-j cells of the LDS region
 #pragma unroll
     for (int m = 0; m < E; ++m)
     {
-        const int j = i + C::T * m;
-        view.put(j, bld<0>(rx, static_cast<uint32_t>(j) * 8u, 0));
+        view.put_at(pad16(i), C::T * m, rx.ld64(static_cast<uint32_t>(i) * 8u, C::T * m * 8u));
     }
     __syncthreads();
     // x'[q]: the row itself for DCT-III, reversed for DST-III (dst3's b[j] takes x[n-1-j] and x[j-1], dct.hpp:160-165)
@@ -182,22 +182,21 @@ __global__ __launch_bounds__((DctCfg<H, E>::threads)) void k_dct_inv(DctArgs a)
 #pragma unroll
     for (int m = E / 2; m < E; ++m)
     {
-        view.put(i2 + C::T * m, v[m]);
+        view.put_at(pad16(i2), C::T * m, v[m]);
     }
     __syncthreads();
-    const __amdgpu_buffer_rsrc_t ry = make_rsrc(a.out + (active ? t * a.odist : 0), row_bytes);
+    const Row<(C::T >= 64)> ry(a.out + (active ? t * a.odist : 0), row_bytes);
     const float sg = SINE ? -1.0f : 1.0f;
 #pragma unroll
     for (int m = 0; m < E / 2; ++m)
     {
-        const int j = i2 + C::T * m;
-        const cf zq = view.get(H - 1 - j);
+        const cf zq = view.get_at(pad16(C::T - 1 - i2), C::T * (E - 1 - m));
         f4v o;
         o.x = v[m].x;
         o.y = sg * zq.y;
         o.z = v[m].y;
         o.w = sg * zq.x;
-        bst128<0>(ry, static_cast<uint32_t>(j) * 16u, 0, o);
+        ry.st128(static_cast<uint32_t>(i2) * 16u, C::T * m * 16u, o);
     }
 }
 

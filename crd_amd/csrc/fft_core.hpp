@@ -71,9 +71,42 @@ template <int STRIDE> struct LdsView
         const int a = pad16(o) * STRIDE;
         return {re[a], re[a + im_off]};
     }
+    // Element o + c for a compile-time c where no carry runs from o's low four bits into c's (o mod 16 + c mod 16 < 16
+    // for the o and c of the call), given p = pad16(o): the pad splits into pad16(o) + pad16(c), so all elements share
+    // one address register and differ in the instruction's offset.
+    __device__ __forceinline__ void put_at(int p, int c, cf v) const
+    {
+        const int a = p * STRIDE;
+        re[a + (c + (c >> 4)) * STRIDE] = v.x;
+        re[a + (c + (c >> 4)) * STRIDE + im_off] = v.y;
+    }
+    __device__ __forceinline__ cf get_at(int p, int c) const
+    {
+        const int a = p * STRIDE;
+        return {re[a + (c + (c >> 4)) * STRIDE], re[a + (c + (c >> 4)) * STRIDE + im_off]};
+    }
 };
 
-template <int N, int E, int P, bool INV, int STRIDE> struct Stage
+// Twiddles of one radix-E stage of a thread (all but W^0).
+template <int E> struct StageTw
+{
+    cf w[E > 1 ? E : 1];
+    __device__ __forceinline__ void load(const cf* __restrict__ t)
+    {
+#pragma unroll
+        for (int j = 1; j < E; ++j)
+        {
+            w[j] = t[j];
+        }
+    }
+};
+
+// AHEAD: a stage's twiddles are loaded before the exchange that leads to it, so that the table's latency passes beside the
+// exchange and the barriers (the loads would otherwise wait for the second barrier). SHARED: one LDS address register for all
+// elements (put_at) in place of one computed each. Together, 2^25 points C2C: n = 512 111 -> 96 us, 8192 138 -> 133, 16384 183 -> 162, 2^17 200 -> 187, 2^20 244 ->
+// 237, 2^22 325 -> 297. Up to 16 values per thread (more would not fit the registers) and from 16 threads per sequence
+// (n = 16 at 4 values, whose table sits in one line: 97 us without, 114 with).
+template <int N, int E, int P, bool INV, int STRIDE, bool AHEAD, bool SHARED> struct Stage
 {
     using G = Geometry<N, E>;
     static constexpr int R = (P == 1) ? G::R0 : E;
@@ -81,8 +114,10 @@ template <int N, int E, int P, bool INV, int STRIDE> struct Stage
     static constexpr int T = G::T;
     static constexpr bool kLast = (static_cast<long>(P) * R == N);
 
-    static __device__ __forceinline__ void run(cf (&v)[E], int i, const LdsView<STRIDE>& lds, const cf* __restrict__ tw)
+    static __device__ __forceinline__ void run(cf (&v)[E], int i, const LdsView<STRIDE>& lds, const cf* __restrict__ tw,
+                                               StageTw<E>& pre)
     {
+        const cf* const next = tw + (P > 1 ? P * R : 0);
 #pragma unroll
         for (int q = 0; q < Q; ++q)
         {
@@ -100,8 +135,12 @@ template <int N, int E, int P, bool INV, int STRIDE> struct Stage
 #pragma unroll
                 for (int j = 1; j < R; ++j)
                 {
-                    a[j] = ctw<INV>(a[j], w[j]);
+                    a[j] = ctw<INV>(a[j], AHEAD ? pre.w[j] : w[j]);
                 }
+            }
+            if constexpr (!kLast && AHEAD && P > 1)
+            {
+                pre.load(next + (i & (P * R - 1)) * E);
             }
             Dft<R, INV>::run(a);
             if constexpr (kLast)
@@ -114,11 +153,19 @@ template <int N, int E, int P, bool INV, int STRIDE> struct Stage
             }
             else
             {
-                const int base = (b - k) * R + k;
+                // base + j P, base = (b - k) R + k: (b - k) R is a multiple of P R and k + j P < P R, so no carry
+                const int base = (b - k) * R + (((b - k) * R) >> 4) + k + (k >> 4);
 #pragma unroll
                 for (int j = 0; j < R; ++j)
                 {
-                    lds.put(base + j * P, a[j]);
+                    if constexpr (SHARED)
+                    {
+                        lds.put_at(base, j * P, a[j]);
+                    }
+                    else
+                    {
+                        lds.put((b - k) * R + k + j * P, a[j]);
+                    }
                 }
             }
         }
@@ -128,20 +175,26 @@ template <int N, int E, int P, bool INV, int STRIDE> struct Stage
 #pragma unroll
             for (int m = 0; m < E; ++m)
             {
-                v[m] = lds.get(i + T * m);
+                v[m] = SHARED ? lds.get_at(pad16(i), T * m) : lds.get(i + T * m); // i < T, a power of two: no carry
             }
             __syncthreads();
-            Stage<N, E, P * R, INV, STRIDE>::run(v, i, lds, tw + (P > 1 ? P * R : 0));
+            Stage<N, E, P * R, INV, STRIDE, AHEAD, SHARED>::run(v, i, lds, next, pre);
         }
     }
 };
 
 // The whole transform: v holds x[i + T*m] on entry and X[i + T*m] on exit. Every thread of the workgroup must
 // call it (it synchronises the workgroup between stages). `tw` is the table of the stages after the first.
-template <int N, int E, bool INV, int STRIDE>
+template <int N, int E, bool INV, int STRIDE, bool AHEAD = (E <= 16 && N / E >= 16), bool SHARED = true>
 __device__ __forceinline__ void fft_core(cf (&v)[E], int i, const LdsView<STRIDE>& lds, const cf* __restrict__ tw)
 {
-    Stage<N, E, 1, INV, STRIDE>::run(v, i, lds, tw);
+    using G = Geometry<N, E>;
+    StageTw<E> pre;
+    if constexpr (AHEAD && N > G::R0)
+    {
+        pre.load(tw + (i & (G::R0 - 1)) * E);
+    }
+    Stage<N, E, 1, INV, STRIDE, AHEAD, SHARED>::run(v, i, lds, tw, pre);
 }
 
 } // namespace crdfft::dev

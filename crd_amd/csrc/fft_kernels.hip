@@ -184,6 +184,7 @@ __global__ __launch_bounds__((RowCfg<N, E>::threads)) void k_rows(RowArgs a)
     using C = RowCfg<N, E>;
     extern __shared__ float lds[];
     const int tid = threadIdx.x;
+    // (the sequence's addresses stay per-lane here: as scalars, n = 4096 x 1024 ran 15.4 us against 14.0)
     const int local = tid / C::T;
     const int i = tid - local * C::T;
     const uint64_t t = static_cast<uint64_t>(blockIdx.x) * C::M + local;
@@ -203,7 +204,12 @@ __global__ __launch_bounds__((RowCfg<N, E>::threads)) void k_rows(RowArgs a)
         }
     }
     const LdsView<1> view{lds + local * C::RS, C::LF};
-    fft_core<N, E, INV, 1>(v, i, view, reinterpret_cast<const cf*>(a.tw));
+    // Twiddles ahead of the exchanges and shared LDS addresses, except for the four 512-thread workgroups a CU holds at n =
+    // 4096: a batch that fills the chip once reads in one burst and writes in another, and what gets its workgroups through
+    // the stages in step makes the bursts meet less (n = 4096 x 1024: 13.7 us without either, 14.1 with the shared addresses,
+    // 16.7 with both; x 256 6.8 / 6.6 / 6.1, x 4096 56.5 / 56.4 / 55.5).
+    constexpr bool kBurst = C::T == 512;
+    fft_core<N, E, INV, 1, E <= 16 && C::T >= 16 && !kBurst, !kBurst>(v, i, view, reinterpret_cast<const cf*>(a.tw));
     if (active)
     {
         store_strided<E>(v, reinterpret_cast<cf*>(a.out) + t * a.odist + i, static_cast<uint32_t>(C::T), a.scale,
@@ -833,12 +839,12 @@ __global__ __launch_bounds__((RowCfg<N, E>::threads)) void k_blue(BlueArgs a)
     using C = RowCfg<N, E>;
     extern __shared__ float lds[];
     const int tid = threadIdx.x;
-    const int local = tid / C::T;
+    const int local = slot_of<C::T>(tid);
     const int i = tid - local * C::T;
     const uint64_t t = static_cast<uint64_t>(blockIdx.x) * C::M + local;
     const bool active = t < a.count;
     const uint32_t bytes = static_cast<uint32_t>(a.n * sizeof(cf));
-    const __amdgpu_buffer_rsrc_t rx = make_rsrc(a.in + (active ? t * a.idist : 0), active ? bytes : 0u);
+    const Row<(C::T >= 64), true> rx(a.in + (active ? t * a.idist : 0), active ? bytes : 0u);
     const __amdgpu_buffer_rsrc_t rc = make_rsrc(a.chirp, bytes);
     const __amdgpu_buffer_rsrc_t rb = make_rsrc(a.bhat, static_cast<uint32_t>(N * sizeof(cf)));
     const uint32_t o0 = static_cast<uint32_t>(i) * sizeof(cf);
@@ -847,7 +853,7 @@ __global__ __launch_bounds__((RowCfg<N, E>::threads)) void k_blue(BlueArgs a)
 #pragma unroll
     for (int m = 0; m < E; ++m)
     {
-        cf x = bld<0>(rx, o0, m * kStep);
+        cf x = rx.ld64(o0, m * kStep);
         if constexpr (INV)
         {
             x.y = -x.y; // IDFT(x) = conj(DFT(conj x)) / n
@@ -873,7 +879,7 @@ __global__ __launch_bounds__((RowCfg<N, E>::threads)) void k_blue(BlueArgs a)
     fft_core<N, E, true, 1>(v, i2, view, tw);
     uint32_t o2 = o0;
     asm volatile("" : "+v"(o2));
-    const __amdgpu_buffer_rsrc_t ry = make_rsrc(a.out + (active ? t * a.odist : 0), active ? bytes : 0u);
+    const Row<(C::T >= 64), true> ry(a.out + (active ? t * a.odist : 0), active ? bytes : 0u);
     const float cm = 1.0f / static_cast<float>(N);
     const float cn = 1.0f / static_cast<float>(a.n);
 #pragma unroll
@@ -887,7 +893,7 @@ __global__ __launch_bounds__((RowCfg<N, E>::threads)) void k_blue(BlueArgs a)
             y.x *= cn;
             y.y = -y.y * cn;
         }
-        bst<0>(ry, o2, m * kStep, y);
+        ry.st64(o2, m * kStep, y);
     }
 }
 

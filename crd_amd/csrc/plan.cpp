@@ -841,12 +841,11 @@ crdfft_status execute_impl(crdfft_plan p, const void* in, void* out, int32_t dir
             int se = 0;
             unsigned per_group = 0;
             if (sh.algorithm == CRDFFT_ALGO_SINGLE && (p->flags & CRDFFT_FLAG_SEPARATE_PASSES) == 0 && !p->floor &&
-                h >= 256 &&
                 crdfft::spec_shape(h, &se, &per_group) && se == sh.e)
             {
-                // 512 <= n <= 32768: load, half-length core, recombine and store in one launch (the spectral
-                // kernel's plain mode: no window, no detrend, frames = rows at idist); measured 1.3-1.7x the
-                // separate passes there, and slower below (a few threads per row load poorly)
+                // n <= 32768: load, half-length core, recombine and store in one launch (the spectral kernel's plain
+                // mode: no window, no detrend, frames = rows at idist); measured 1.2-2.1x the separate passes (2^25
+                // points: n = 4 124 / 148 us, 16 105 / 115, 64 51 / 99, 256 46 / 93)
                 const crdfft::SpecArgs a{static_cast<const float*>(in), nullptr, p->wreal.as<cfloat>(),
                                          p->tw_single.as<cfloat>(), out, sh.batch, p->idist, 1.0f, 0, p->odist};
                 CRDFFT_TRY(prof.before());
@@ -889,11 +888,10 @@ crdfft_status execute_impl(crdfft_plan p, const void* in, void* out, int32_t dir
             const uint64_t h = sh.n / 2;
             cfloat* o = static_cast<cfloat*>(out);
             if (sh.algorithm == CRDFFT_ALGO_SINGLE && (p->flags & CRDFFT_FLAG_SEPARATE_PASSES) == 0 && !p->floor &&
-                h >= 512 &&
                 crdfft::c2r_one_kernel_e(h) == sh.e)
             {
-                // 1024 <= n <= 32768: recombine, inverse half-length core and store in one launch (1.1-1.4x the
-                // separate passes there, slower below)
+                // n <= 32768: recombine, inverse half-length core and store in one launch; measured 1.2-1.9x the
+                // separate passes (2^25 points: n = 4 54 / 100 us, 32 65 / 89, 128 45 / 84, 512 47 / 85)
                 const crdfft::C2rArgs a{static_cast<const cfloat*>(in), o, p->wreal.as<cfloat>(),
                                         p->tw_single.as<cfloat>(), sh.batch, p->idist, p->odist / 2,
                                         1.0f / static_cast<float>(h)};

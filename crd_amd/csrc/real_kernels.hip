@@ -101,28 +101,28 @@ __global__ __launch_bounds__((C2rCfg<H, E>::threads)) void k_c2r1(C2rArgs a)
     using C = C2rCfg<H, E>;
     extern __shared__ float lds[];
     const int tid = threadIdx.x;
-    const int local = tid / C::T;
+    const int local = slot_of<C::T>(tid);
     const int i = tid - local * C::T;
     const uint64_t t = static_cast<uint64_t>(blockIdx.x) * C::M + local;
     const bool active = t < a.count;
-    const __amdgpu_buffer_rsrc_t rx =
-        make_rsrc(reinterpret_cast<const cf*>(a.in) + (active ? t * a.idist : 0), active ? (H + 1) * 8u : 0u);
+    const Row<(C::T >= 64)> rx(reinterpret_cast<const cf*>(a.in) + (active ? t * a.idist : 0),
+                               active ? (H + 1) * 8u : 0u);
     const __amdgpu_buffer_rsrc_t rw = make_rsrc(a.w, (H + 1) * 8u);
     cf v[E];
 #pragma unroll
     for (int m = 0; m < E; ++m)
     {
-        const uint32_t k = static_cast<uint32_t>(i + C::T * m);
-        v[m] = c2r_z(bld<0>(rx, 8u * k, 0), bld<0>(rx, 8u * (H - k), 0), bld<0>(rw, 8u * k, 0), a.scale);
+        const uint32_t k = 8u * static_cast<uint32_t>(i), step = 8u * C::T * m; // slot k = i + T m, in bytes
+        v[m] = c2r_z(rx.ld64(k, step), rx.ld64(8u * (H - C::T * (E - 1)) - k, 8u * C::T * (E - 1) - step),
+                     bld<0>(rw, k, step), a.scale);
     }
     const LdsView<1> view{lds + local * C::RS, C::LF};
     fft_core<H, E, true, 1>(v, i, view, reinterpret_cast<const cf*>(a.tw));
-    const __amdgpu_buffer_rsrc_t ry =
-        make_rsrc(reinterpret_cast<cf*>(a.out) + (active ? t * a.odist : 0), active ? H * 8u : 0u);
+    const Row<(C::T >= 64)> ry(reinterpret_cast<cf*>(a.out) + (active ? t * a.odist : 0), active ? H * 8u : 0u);
 #pragma unroll
     for (int m = 0; m < E; ++m)
     {
-        bst<0>(ry, 8u * static_cast<uint32_t>(i + C::T * m), 0, v[m]);
+        ry.st64(8u * static_cast<uint32_t>(i), 8u * C::T * m, v[m]);
     }
 }
 

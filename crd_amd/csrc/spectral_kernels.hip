@@ -49,7 +49,7 @@ __global__ __launch_bounds__((SpecCfg<H, E>::threads)) void k_spec(SpecArgs a)
     constexpr int T = C::T;
     extern __shared__ float lds[];
     const int tid = threadIdx.x;
-    const int local = tid / T;
+    const int local = slot_of<T>(tid);
     const int i = tid - local * T;
     const LdsView<1> view{lds + local * C::RS, C::LF};
     float* red = lds + C::RS * C::M;
@@ -73,22 +73,25 @@ __global__ __launch_bounds__((SpecCfg<H, E>::threads)) void k_spec(SpecArgs a)
     {
         const uint64_t f = group + it * groups;
         const bool active = f < a.frames;
-        // the tables are the same for every frame; an empty asm hides that, so the compiler reloads them per frame
+        // the tables are the same for every frame; an empty asm hides that from the frame loop, so the compiler reloads them per frame
         // (L1/L2 hits) instead of holding every butterfly's twiddles in registers across the frame loop
         const cf* tw = reinterpret_cast<const cf*>(a.tw);
         const cf* wk = reinterpret_cast<const cf*>(a.wtab);
         const float* win = a.window;
-        asm volatile("" : "+s"(tw), "+s"(wk), "+s"(win));
+        if constexpr (MODE == 2)
+        {
+            asm volatile("" : "+s"(tw), "+s"(wk), "+s"(win));
+        }
         // the frame through a buffer resource: an inactive frame gets no records, so its loads read zeros and touch
         // no memory
-        const __amdgpu_buffer_rsrc_t xr = make_rsrc(a.x + (active ? f * a.hop : 0), active ? 8u * H : 0u);
+        const Row<(T >= 64)> xr(a.x + (active ? f * a.hop : 0), active ? 8u * H : 0u);
         cf v[E];
         if (pairs)
         {
 #pragma unroll
             for (int m = 0; m < E; ++m)
             {
-                v[m] = bld<0>(xr, 8u * static_cast<uint32_t>(i + T * m), 0);
+                v[m] = xr.ld64(8u * static_cast<uint32_t>(i), 8u * T * m);
             }
         }
         else
@@ -96,8 +99,8 @@ __global__ __launch_bounds__((SpecCfg<H, E>::threads)) void k_spec(SpecArgs a)
 #pragma unroll
             for (int m = 0; m < E; ++m)
             {
-                const uint32_t j = static_cast<uint32_t>(i + T * m);
-                v[m] = cf{bld32<0>(xr, 8u * j, 0), bld32<0>(xr, 8u * j + 4u, 0)};
+                const uint32_t j = 8u * static_cast<uint32_t>(i);
+                v[m] = cf{xr.ld32(j, 8u * T * m), xr.ld32(j + 4u, 8u * T * m)};
             }
         }
         if (a.detrend != 0)
@@ -158,7 +161,7 @@ __global__ __launch_bounds__((SpecCfg<H, E>::threads)) void k_spec(SpecArgs a)
 #pragma unroll
         for (int m = 0; m < E; ++m)
         {
-            view.put(i + T * m, v[m]);
+            view.put_at(pad16(i), T * m, v[m]);
         }
         __syncthreads();
         // recombine and epilogue per slot (nothing but the accumulators outlives the frame)
@@ -168,7 +171,10 @@ __global__ __launch_bounds__((SpecCfg<H, E>::threads)) void k_spec(SpecArgs a)
         {
             const int k = i + T * m;
             const cf zk = v[m];
-            const cf zh = view.get(k == 0 ? 0 : H - k);
+            // element H - k = (T - i) + T (E - 1 - m): pads apart, as T - i carries into no higher part for i > 0; slot 0 is
+            // its own mirror
+            const cf zh = m == 0 ? view.get(k == 0 ? 0 : H - k)
+                                 : (T >= 16 ? view.get_at(pad16(T - i), T * (E - 1 - m)) : view.get(H - k));
             const cf e = {(zk.x + zh.x) * 0.5f, (zk.y - zh.y) * 0.5f};
             const cf o = {(zk.y + zh.y) * 0.5f, (zh.x - zk.x) * 0.5f};
             const cf xk = cadd(e, cmul(o, wk[k]));
@@ -180,7 +186,7 @@ __global__ __launch_bounds__((SpecCfg<H, E>::threads)) void k_spec(SpecArgs a)
                 {
                     cf* out = reinterpret_cast<cf*>(a.out) + row;
                     out[k] = xk;
-                    if (k == 0)
+                    if (m == 0 && k == 0)
                     {
                         out[H] = xn;
                     }
@@ -188,7 +194,7 @@ __global__ __launch_bounds__((SpecCfg<H, E>::threads)) void k_spec(SpecArgs a)
             }
             else
             {
-                const float p = a.scale * (xk.x * xk.x + xk.y * xk.y) * (k == 0 ? 1.0f : 2.0f);
+                const float p = a.scale * (xk.x * xk.x + xk.y * xk.y) * (m == 0 && k == 0 ? 1.0f : 2.0f);
                 const float pn = a.scale * (xn.x * xn.x);
                 if constexpr (MODE == 1)
                 {
@@ -196,7 +202,7 @@ __global__ __launch_bounds__((SpecCfg<H, E>::threads)) void k_spec(SpecArgs a)
                     {
                         float* out = reinterpret_cast<float*>(a.out) + row;
                         out[k] = p;
-                        if (k == 0)
+                        if (m == 0 && k == 0)
                         {
                             out[H] = pn;
                         }
@@ -205,7 +211,7 @@ __global__ __launch_bounds__((SpecCfg<H, E>::threads)) void k_spec(SpecArgs a)
                 else
                 {
                     acc[m] += active ? p : 0.0f;
-                    if (k == 0)
+                    if (m == 0 && k == 0)
                     {
                         acc[E] += active ? pn : 0.0f;
                     }
