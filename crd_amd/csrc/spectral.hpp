@@ -32,6 +32,12 @@ bool spec_shape(uint64_t h, int* e, unsigned* frames_per_group);
 hipError_t launch_spec(uint64_t h, int mode, const SpecArgs& a, uint64_t groups, hipStream_t s);
 // Resident workgroups per CU of the Welch lane-group kernel (the persistent grid is this times the CU count).
 hipError_t spec_welch_residency(uint64_t h, int* per_cu);
+// Welch over pairs of frames (k_welch): values per thread and pairs per workgroup for frames of n samples (false: no
+// instantiation), the launch (a.tw: the stage twiddles of (n, e); a.out: one partial row per pair slot of the grid) and
+// the resident workgroups per CU.
+bool welch_pair_shape(uint64_t n, int* e, unsigned* pairs_per_group);
+hipError_t launch_welch_pairs(uint64_t n, const SpecArgs& a, uint64_t groups, hipStream_t s);
+hipError_t welch_pair_residency(uint64_t n, int* per_cu);
 // acc[k] = ((first ? 0 : acc[k]) + rows[0][k] + ... + rows[nrows-1][k]) * scale, summed in a fixed order.
 hipError_t launch_spec_sum(const float* rows, float* acc, uint64_t nfreq, uint64_t nrows, bool first, float scale,
                            hipStream_t s);

@@ -236,45 +236,205 @@ __global__ __launch_bounds__((SpecCfg<H, E>::threads)) void k_spec(SpecArgs a)
     }
 }
 
+// k_welch<N, E>: the Welch sum over pairs of frames. Frames 2 p and 2 p + 1 are the real and imaginary parts of one
+// N-point transform Z, and |A[k]|^2 + |B[k]|^2 = (|Z[k]|^2 + |Z[N-k]|^2) / 2, so nothing has to be told apart per
+// frame: a lane group of T = N/E threads adds scale |Z[k]|^2 of its pairs g, g + G, ... to its E slots, folds k onto
+// N - k through LDS once at the end and the workgroup writes one partial row of N/2 + 1 densities. Per frame that is half an N-point
+// transform (12 levels of 4096 points for two frames) in place of a half-length one, a recombine and its LDS exchange.
+// Bound by the vector unit (about 900 instructions a thread and pair at N = 4096, E = 16; floor by bytes 44 us). Measured,
+// 2^26 samples at 50 % overlap: N = 4096 268 -> 170 us, 1024 200 -> 112, 256 303 -> 97, 64 683 -> 88. Loading the next pair
+// ahead (32 more registers) measured no better, nor did reloading the twiddles per pair instead of keeping them.
+template <int N, int E> struct WelchCfg
+{
+    static constexpr int T = N / E;
+    static constexpr int M = T >= 256 ? 1 : 256 / T; // pairs per workgroup
+    static constexpr int threads = T * M;
+    static constexpr int LF = lds_floats(N);
+    static constexpr int RS = round_up(2 * LF, 64) + (T < 64 ? T : 0); // per-pair region (re then im)
+    static constexpr int lds_bytes = (RS * M + 2 * threads / 64 + 2) * 4;
+};
+
+template <int N, int E>
+__global__ __launch_bounds__((WelchCfg<N, E>::threads)) void k_welch(SpecArgs a)
+{
+    using C = WelchCfg<N, E>;
+    constexpr int T = C::T;
+    extern __shared__ float lds[];
+    const int tid = threadIdx.x;
+    const int local = slot_of<T>(tid);
+    const int i = tid - local * T;
+    const LdsView<1> view{lds + local * C::RS, C::LF};
+    float* red = lds + C::RS * C::M;
+    const uint64_t group = static_cast<uint64_t>(blockIdx.x) * C::M + local;
+    const uint64_t groups = static_cast<uint64_t>(gridDim.x) * C::M;
+    const uint64_t pairs = (a.frames + 1) / 2;
+    const uint64_t iters = (pairs + groups - 1) / groups; // the same for every lane group: idle ones read no records
+    float acc[E];
+#pragma unroll
+    for (int m = 0; m < E; ++m)
+    {
+        acc[m] = 0.0f;
+    }
+    const __amdgpu_buffer_rsrc_t wr = make_rsrc(a.window, a.window != nullptr ? 4u * N : 0u);
+    const uint32_t o4 = 4u * static_cast<uint32_t>(i);
+    auto load = [&](cf (&d)[E], uint64_t it) {
+        const uint64_t f = 2 * (group + it * groups);
+        const bool one = f < a.frames, two = f + 1 < a.frames;
+        const Row<(T >= 64)> ra(a.x + (one ? f * a.hop : 0), one ? 4u * N : 0u);
+        const Row<(T >= 64)> rb(a.x + (two ? (f + 1) * a.hop : 0), two ? 4u * N : 0u);
+#pragma unroll
+        for (int m = 0; m < E; ++m)
+        {
+            d[m] = cf{ra.ld32(o4, 4u * T * m), rb.ld32(o4, 4u * T * m)};
+            if constexpr (T < 64)
+            {
+                d[m] = cf{one ? d[m].x : 0.0f, two ? d[m].y : 0.0f};
+            }
+        }
+    };
+    float win[E];
+#pragma unroll
+    for (int m = 0; m < E; ++m)
+    {
+        win[m] = a.window != nullptr ? bld32<0>(wr, o4, 4u * T * m) : 1.0f;
+    }
+#pragma unroll 1
+    for (uint64_t it = 0; it < iters; ++it)
+    {
+        cf v[E];
+        load(v, it);
+        if (a.detrend != 0)
+        {
+            // both means in a fixed order: lane butterflies within a wave, then the waves' sums in wave order
+            cf part = {0.0f, 0.0f};
+#pragma unroll
+            for (int m = 0; m < E; ++m)
+            {
+                part = cadd(part, v[m]);
+            }
+            constexpr int W = T < 64 ? T : 64;
+#pragma unroll
+            for (int o = W / 2; o > 0; o >>= 1)
+            {
+                part.x += __shfl_xor(part.x, o, 64);
+                part.y += __shfl_xor(part.y, o, 64);
+            }
+            if constexpr (T > 64)
+            {
+                cf* const sums = reinterpret_cast<cf*>(red);
+                if ((tid & 63) == 0)
+                {
+                    sums[tid >> 6] = part;
+                }
+                __syncthreads();
+                part = cf{0.0f, 0.0f};
+#pragma unroll
+                for (int w = 0; w < T / 64; ++w)
+                {
+                    part = cadd(part, sums[((local * T) >> 6) + w]);
+                }
+            }
+            const cf mean = {part.x / static_cast<float>(N), part.y / static_cast<float>(N)};
+#pragma unroll
+            for (int m = 0; m < E; ++m)
+            {
+                v[m] = csub(v[m], mean);
+            }
+        }
+        if (a.window != nullptr)
+        {
+#pragma unroll
+            for (int m = 0; m < E; ++m)
+            {
+                v[m].x *= win[m];
+                v[m].y *= win[m];
+            }
+        }
+        fft_core<N, E, false, 1>(v, i, view, reinterpret_cast<const cf*>(a.tw));
+        // an idle lane group or half of a pair: the samples are zeros, less a mean of zero
+#pragma unroll
+        for (int m = 0; m < E; ++m)
+        {
+            acc[m] += a.scale * (v[m].x * v[m].x + v[m].y * v[m].y);
+        }
+    }
+    // the lane groups' sums in group order, k folded onto N - k: P[k] = S[k] + S[N - k] (the one-sided doubling of the
+    // halves), P[0] and P[N/2] alone; one partial row per workgroup
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < E; ++m)
+    {
+        lds[local * N + i + T * m] = acc[m];
+    }
+    __syncthreads();
+    float* prow = reinterpret_cast<float*>(a.out) + static_cast<uint64_t>(blockIdx.x) * (N / 2 + 1);
+    for (int k = tid; k <= N / 2; k += C::threads)
+    {
+        float p = 0.0f;
+#pragma unroll 4
+        for (int g = 0; g < C::M; ++g)
+        {
+            p += lds[g * N + k] + (k == 0 || k == N / 2 ? 0.0f : lds[g * N + N - k]);
+        }
+        prow[k] = p;
+    }
+}
+
 // acc[k] = ((first ? 0 : acc[k]) + sum over the rows of rows[r][k]) * scale, in a fixed order: a workgroup owns 64
 // bins, its 16 row groups sum rows g, g + 16, ... (four loads in flight per step), and the 16 partial sums are added
-// in group order, so the result does not depend on timing.
+// in group order, so the result does not depend on timing. The sums carry their rounding errors along, so thousands of
+// rows add none of their own.
 constexpr int kSumBins = 64;
 constexpr int kSumGroups = 16;
+
+// s += x, the rounding error collected in c (Knuth's two-sum)
+__device__ __forceinline__ void add_compensated(float& s, float& c, float x)
+{
+    const float t = s + x;
+    const float b = t - s;
+    c += (s - (t - b)) + (x - b);
+    s = t;
+}
 
 __global__ __launch_bounds__(kSumBins * kSumGroups) void k_spec_sum(const float* rows, float* acc, uint64_t nfreq,
                                                                     uint64_t nrows, int first, float scale)
 {
-    __shared__ float part[kSumGroups][kSumBins];
+    __shared__ float part[kSumGroups][kSumBins], rest[kSumGroups][kSumBins];
     const int kk = threadIdx.x % kSumBins;
     const int g = threadIdx.x / kSumBins;
     const uint64_t k = static_cast<uint64_t>(blockIdx.x) * kSumBins + kk;
-    float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f, s3 = 0.0f;
+    float s = 0.0f, c = 0.0f;
     if (k < nfreq)
     {
         uint64_t r = g;
         for (; r + 3 * kSumGroups < nrows; r += 4 * kSumGroups)
         {
-            s0 += rows[r * nfreq + k];
-            s1 += rows[(r + kSumGroups) * nfreq + k];
-            s2 += rows[(r + 2 * kSumGroups) * nfreq + k];
-            s3 += rows[(r + 3 * kSumGroups) * nfreq + k];
+            const float x0 = rows[r * nfreq + k], x1 = rows[(r + kSumGroups) * nfreq + k];
+            const float x2 = rows[(r + 2 * kSumGroups) * nfreq + k], x3 = rows[(r + 3 * kSumGroups) * nfreq + k];
+            add_compensated(s, c, x0);
+            add_compensated(s, c, x1);
+            add_compensated(s, c, x2);
+            add_compensated(s, c, x3);
         }
         for (; r < nrows; r += kSumGroups)
         {
-            s0 += rows[r * nfreq + k];
+            add_compensated(s, c, rows[r * nfreq + k]);
         }
     }
-    part[g][kk] = (s0 + s1) + (s2 + s3);
+    part[g][kk] = s;
+    rest[g][kk] = c;
     __syncthreads();
     if (g == 0 && k < nfreq)
     {
-        float s = first != 0 ? 0.0f : acc[k];
+        s = first != 0 ? 0.0f : acc[k];
+        c = 0.0f;
         for (int q = 0; q < kSumGroups; ++q)
         {
-            s += part[q][kk];
+            add_compensated(s, c, part[q][kk]);
+            c += rest[q][kk];
         }
-        acc[k] = s * scale;
+        // a sum that has left the range of the type has no rest (inf - inf)
+        acc[k] = (c - c == 0.0f ? s + c : s) * scale;
     }
 }
 
@@ -283,6 +443,12 @@ __global__ __launch_bounds__(kSumBins * kSumGroups) void k_spec_sum(const float*
 #define CRDFFT_SPEC_LIST(X)                                                                                            \
     X(2, 2) X(4, 4) X(8, 8) X(16, 4) X(32, 4) X(64, 4) X(128, 4) X(256, 4) X(512, 8) X(1024, 8) X(2048, 8) X(4096, 8)  \
         X(8192, 8) X(16384, 16)
+
+// (N, E) of the pair kernel: the fastest per length over a 2^26-sample signal at 50 % overlap (us at E = 8 / 16 / 32; 4
+// values per thread were slower still): 64 87 / - / -, 128 108 / 107 / -, 256 116 / 97 / -, 512 114 / 131 / 106,
+// 1024 151 / 158 / 112, 2048 155 / 161 / 153, 4096 170 / 168 / 167, 8192 - / 226 / 198.
+#define CRDFFT_WELCH_LIST(X)                                                                                           \
+    X(8, 4) X(16, 8) X(32, 8) X(64, 8) X(128, 16) X(256, 16) X(512, 32) X(1024, 32) X(2048, 32) X(4096, 16) X(8192, 32)
 
 template <typename K> hipError_t set_lds(K kernel, unsigned bytes)
 {
@@ -348,6 +514,55 @@ hipError_t spec_welch_residency(uint64_t h, int* per_cu)
         return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, kern, C::threads, C::lds_bytes);                   \
     }
     CRDFFT_SPEC_LIST(X)
+#undef X
+    return hipErrorInvalidValue;
+}
+
+bool welch_pair_shape(uint64_t n, int* e, unsigned* pairs_per_group)
+{
+#define X(N, E)                                                                                                        \
+    if (n == N)                                                                                                        \
+    {                                                                                                                  \
+        *e = E;                                                                                                        \
+        *pairs_per_group = WelchCfg<N, E>::M;                                                                          \
+        return true;                                                                                                   \
+    }
+    CRDFFT_WELCH_LIST(X)
+#undef X
+    return false;
+}
+
+hipError_t launch_welch_pairs(uint64_t n, const SpecArgs& a, uint64_t groups, hipStream_t s)
+{
+#define X(N, E)                                                                                                        \
+    if (n == N)                                                                                                        \
+    {                                                                                                                  \
+        using C = WelchCfg<N, E>;                                                                                      \
+        hipError_t err = set_lds(k_welch<N, E>, C::lds_bytes);                                                         \
+        if (err != hipSuccess)                                                                                         \
+            return err;                                                                                                \
+        if (groups == 0 || groups > 0xFFFFFFFFull)                                                                     \
+            return hipErrorInvalidValue;                                                                               \
+        hipLaunchKernelGGL((k_welch<N, E>), dim3(static_cast<unsigned>(groups)), dim3(C::threads), C::lds_bytes, s, a); \
+        return hipGetLastError();                                                                                      \
+    }
+    CRDFFT_WELCH_LIST(X)
+#undef X
+    return hipErrorInvalidValue;
+}
+
+hipError_t welch_pair_residency(uint64_t n, int* per_cu)
+{
+#define X(N, E)                                                                                                        \
+    if (n == N)                                                                                                        \
+    {                                                                                                                  \
+        using C = WelchCfg<N, E>;                                                                                      \
+        const hipError_t err = set_lds(k_welch<N, E>, C::lds_bytes);                                                   \
+        if (err != hipSuccess)                                                                                         \
+            return err;                                                                                                \
+        return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, k_welch<N, E>, C::threads, C::lds_bytes);          \
+    }
+    CRDFFT_WELCH_LIST(X)
 #undef X
     return hipErrorInvalidValue;
 }
