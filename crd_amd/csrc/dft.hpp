@@ -223,7 +223,7 @@ template <bool INV> struct Dft<7, INV> : DftOdd<7, INV>
 
 // R = R1 * R2 in registers: R2 DFTs of size R1 over x[R2 n1 + n2], twiddle W_R^{n2 k1}, R1 DFTs of size R2,
 // output X[k1 + R1 k2].
-template <int R1, int R2, bool INV> struct DftSplit
+template <int R1, int R2, bool INV, class First = Dft<R1, INV>> struct DftSplit
 {
     static constexpr int R = R1 * R2;
     template <int N2, int K1> static __device__ __forceinline__ cf tw(cf a) { return twc<static_cast<long>(N2) * K1, R, INV>(a); }
@@ -246,9 +246,9 @@ template <int R1, int R2, bool INV> struct DftSplit
 #pragma unroll
             for (int n1 = 0; n1 < R1; ++n1)
             {
-                t[n2][n1] = a[R2 * n1 + n2];
+                t[n2][n1] = a[R2 * n1 + n2]; // (a zero half's are not read again)
             }
-            Dft<R1, INV>::run(t[n2]);
+            First::run(t[n2]);
         }
         twall(t, std::make_integer_sequence<int, R2>{});
 #pragma unroll
@@ -282,6 +282,34 @@ template <bool INV> struct Dft<32, INV> : DftSplit<8, 4, INV>
 template <bool INV> struct Dft<64, INV> : DftSplit<8, 8, INV>
 {
 };
+// The DFT of R values (R = 2, 4, 8, 16) whose upper half a[R/2..R) is zero and need not be set: the butterflies that would
+// add those zeros are left out.
+template <int R, bool INV> struct DftHalf;
+
+template <bool INV> struct DftHalf<2, INV>
+{
+    static __device__ __forceinline__ void run(cf* a) { a[1] = a[0]; }
+};
+
+template <bool INV> struct DftHalf<4, INV>
+{
+    static __device__ __forceinline__ void run(cf* a)
+    {
+        const cf x = a[0], y = a[1], z = mul_w4<INV>(a[1]);
+        a[0] = cadd(x, y);
+        a[2] = csub(x, y);
+        a[1] = cadd(x, z);
+        a[3] = csub(x, z);
+    }
+};
+
+template <bool INV> struct DftHalf<8, INV> : DftSplit<2, 4, INV, DftHalf<2, INV>>
+{
+};
+template <bool INV> struct DftHalf<16, INV> : DftSplit<4, 4, INV, DftHalf<4, INV>>
+{
+};
+
 template <bool INV> struct Dft<6, INV> : DftSplit<2, 3, INV>
 {
 };

@@ -106,7 +106,7 @@ template <int E> struct StageTw
 // elements (put_at) in place of one computed each. Together, 2^25 points C2C: n = 512 111 -> 96 us, 8192 138 -> 133, 16384 183 -> 162, 2^17 200 -> 187, 2^20 244 ->
 // 237, 2^22 325 -> 297. Up to 16 values per thread (more would not fit the registers) and from 16 threads per sequence
 // (n = 16 at 4 values, whose table sits in one line: 97 us without, 114 with).
-template <int N, int E, int P, bool INV, int STRIDE, bool AHEAD, bool SHARED> struct Stage
+template <int N, int E, int P, bool INV, int STRIDE, bool AHEAD, bool SHARED, bool HALF = false> struct Stage
 {
     using G = Geometry<N, E>;
     static constexpr int R = (P == 1) ? G::R0 : E;
@@ -125,7 +125,7 @@ template <int N, int E, int P, bool INV, int STRIDE, bool AHEAD, bool SHARED> st
             const int k = b & (P - 1);
             cf a[R];
 #pragma unroll
-            for (int j = 0; j < R; ++j)
+            for (int j = 0; j < (HALF ? R / 2 : R); ++j)
             {
                 a[j] = v[q + j * Q];
             }
@@ -142,7 +142,14 @@ template <int N, int E, int P, bool INV, int STRIDE, bool AHEAD, bool SHARED> st
             {
                 pre.load(next + (i & (P * R - 1)) * E);
             }
-            Dft<R, INV>::run(a);
+            if constexpr (HALF)
+            {
+                DftHalf<R, INV>::run(a);
+            }
+            else
+            {
+                Dft<R, INV>::run(a);
+            }
             if constexpr (kLast)
             {
 #pragma unroll
@@ -184,8 +191,10 @@ template <int N, int E, int P, bool INV, int STRIDE, bool AHEAD, bool SHARED> st
 };
 
 // The whole transform: v holds x[i + T*m] on entry and X[i + T*m] on exit. Every thread of the workgroup must
-// call it (it synchronises the workgroup between stages). `tw` is the table of the stages after the first.
-template <int N, int E, bool INV, int STRIDE, bool AHEAD = (E <= 16 && N / E >= 16), bool SHARED = true>
+// call it (it synchronises the workgroup between stages). `tw` is the table of the stages after the first. HALF: the upper
+// half of the input, v[E/2..E), is zero and not read (E <= 16).
+template <int N, int E, bool INV, int STRIDE, bool AHEAD = (E <= 16 && N / E >= 16), bool SHARED = true,
+          bool HALF = false>
 __device__ __forceinline__ void fft_core(cf (&v)[E], int i, const LdsView<STRIDE>& lds, const cf* __restrict__ tw)
 {
     using G = Geometry<N, E>;
@@ -194,7 +203,7 @@ __device__ __forceinline__ void fft_core(cf (&v)[E], int i, const LdsView<STRIDE
     {
         pre.load(tw + (i & (G::R0 - 1)) * E);
     }
-    Stage<N, E, 1, INV, STRIDE, AHEAD, SHARED>::run(v, i, lds, tw, pre);
+    Stage<N, E, 1, INV, STRIDE, AHEAD, SHARED, HALF>::run(v, i, lds, tw, pre);
 }
 
 } // namespace crdfft::dev

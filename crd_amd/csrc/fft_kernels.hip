@@ -833,6 +833,10 @@ __global__ __launch_bounds__(TH) void k_fused(FusedArgs a)
 // LDS: the only HBM traffic is x in and X out (n points each) plus the L2-resident c and FFT_m(b) tables. The
 // zero padding and the k < n store guard are the buffer resources' range checks: reads at or past n return 0 and
 // writes there are dropped, as are all accesses of an inactive slot (num_records 0).
+// n <= N / 2, so the upper half of a thread's slots is padding on the way in and past the end on the way out: it is never
+// loaded, the first stage leaves out the butterflies that would add it (DftHalf), and the second transform's last stage
+// forms only the lower half (2^23 points: n = 127 67 -> 52 us, 1009 89 -> 76, 4001 113 -> 99). Bound by the vector unit and
+// LDS: two N-point transforms for n points, 4x the floor of its bytes at n = 1009. 16 values per thread: 1009 90 us.
 template <int N, int E, bool INV>
 __global__ __launch_bounds__((RowCfg<N, E>::threads)) void k_blue(BlueArgs a)
 {
@@ -851,7 +855,7 @@ __global__ __launch_bounds__((RowCfg<N, E>::threads)) void k_blue(BlueArgs a)
     constexpr uint32_t kStep = C::T * sizeof(cf);
     cf v[E];
 #pragma unroll
-    for (int m = 0; m < E; ++m)
+    for (int m = 0; m < E / 2; ++m) // n <= N / 2: the upper half is the zero padding
     {
         cf x = rx.ld64(o0, m * kStep);
         if constexpr (INV)
@@ -862,7 +866,7 @@ __global__ __launch_bounds__((RowCfg<N, E>::threads)) void k_blue(BlueArgs a)
     }
     const LdsView<1> view{lds + local * C::RS, C::LF};
     const cf* tw = reinterpret_cast<const cf*>(a.tw);
-    fft_core<N, E, false, 1>(v, i, view, tw);
+    fft_core<N, E, false, 1, (E <= 16 && C::T >= 16), true, true>(v, i, view, tw);
     // the table offsets pass through an empty asm after each transform, so the compiler cannot issue the table
     // loads early and hold them in registers across the transform (at m = 16384 that spills)
     uint32_t o1 = o0;
@@ -883,7 +887,7 @@ __global__ __launch_bounds__((RowCfg<N, E>::threads)) void k_blue(BlueArgs a)
     const float cm = 1.0f / static_cast<float>(N);
     const float cn = 1.0f / static_cast<float>(a.n);
 #pragma unroll
-    for (int m = 0; m < E; ++m)
+    for (int m = 0; m < E / 2; ++m)
     {
         cf y = cmulc(v[m], bld<0>(rc, o2, m * kStep));
         y.x *= cm;
