@@ -81,7 +81,10 @@ typedef enum crdfft_algorithm
 {
     CRDFFT_ALGO_COPY = 0,       /* n == 1 */
     CRDFFT_ALGO_SINGLE = 1,     /* one LDS-staged kernel per transform (n <= 16384) */
-    CRDFFT_ALGO_FOUR_STEP = 2,  /* n = n1*n2: column pass with twiddle, row pass with transposed store */
+    CRDFFT_ALGO_FOUR_STEP = 2,  /* n = n1*n2: column pass with twiddle, row pass with transposed store. Plans of 2^15 and
+                                   2^16 complex points (C2C; R2C / C2R of 2^16) without tuning run both steps of a
+                                   transform on one CU in one launch for as much of the batch as fills the device
+                                   (crdfft_phase_times: phase 0), the two passes for the rest */
     CRDFFT_ALGO_REFERENCE = 3,  /* the radix-2 reference only */
     CRDFFT_ALGO_BLUESTEIN = 4,  /* chirp-z over a power-of-two plan of m >= 2n-1 (any n) */
     CRDFFT_ALGO_FUSED = 5,      /* n = n1*n2 <= 2^17: both four-step passes of a transform in one workgroup of a
@@ -392,8 +395,8 @@ CRDFFT_API crdfft_status crdfft_stft(crdfft_spectral_plan plan, const float* x, 
 CRDFFT_API crdfft_status crdfft_spectrogram(crdfft_spectral_plan plan, const float* x, uint64_t len, double fs,
                                             float* out, void* stream);
 /* welch_psd (spectral.hpp:140-172): psd = nperseg/2+1 floats, the frames' density periodograms averaged. The sum runs
- * in a fixed order (lane-group partial rows, then strided row groups added in group order), so the result is bit-identical run to run. Uses
- * the plan's scratch for the partial rows (per stream). All zeros when there is no frame. */
+ * in a fixed order (partial rows of lane groups, two frames at a time from 512 (1024 above 256 samples a frame) frames on,
+ * then strided row groups added in group order), so the result is bit-identical run to run. Uses the plan's scratch for the partial rows (per stream). All zeros when there is no frame. */
 CRDFFT_API crdfft_status crdfft_welch(crdfft_spectral_plan plan, const float* x, uint64_t len, double fs, float* psd,
                                       void* stream);
 
