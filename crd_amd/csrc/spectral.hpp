@@ -39,7 +39,8 @@ bool welch_pair_shape(uint64_t n, int* e, unsigned* pairs_per_group);
 hipError_t launch_welch_pairs(uint64_t n, const SpecArgs& a, uint64_t groups, hipStream_t s);
 hipError_t welch_pair_residency(uint64_t n, int* per_cu);
 // acc[k] = ((first ? 0 : acc[k]) + rows[0][k] + ... + rows[nrows-1][k]) * scale, summed in a fixed order.
+// scale_lo: what rounding left of the scale.
 hipError_t launch_spec_sum(const float* rows, float* acc, uint64_t nfreq, uint64_t nrows, bool first, float scale,
-                           hipStream_t s);
+                           hipStream_t s, float scale_lo = 0.0f);
 
 } // namespace crdfft

@@ -397,7 +397,7 @@ __device__ __forceinline__ void add_compensated(float& s, float& c, float x)
 }
 
 __global__ __launch_bounds__(kSumBins * kSumGroups) void k_spec_sum(const float* rows, float* acc, uint64_t nfreq,
-                                                                    uint64_t nrows, int first, float scale)
+                                                                    uint64_t nrows, int first, float scale, float scale_lo)
 {
     __shared__ float part[kSumGroups][kSumBins], rest[kSumGroups][kSumBins];
     const int kk = threadIdx.x % kSumBins;
@@ -433,8 +433,9 @@ __global__ __launch_bounds__(kSumBins * kSumGroups) void k_spec_sum(const float*
             add_compensated(s, c, part[q][kk]);
             c += rest[q][kk];
         }
-        // a sum that has left the range of the type has no rest (inf - inf)
-        acc[k] = (c - c == 0.0f ? s + c : s) * scale;
+        // (s + c) (scale + scale_lo) rounded once; a sum that has left the range of the type has no rest (inf - inf)
+        const float plain = (c - c == 0.0f ? s + c : s) * scale;
+        acc[k] = plain - plain == 0.0f ? __fmaf_rn(s, scale, __fmaf_rn(c, scale, s * scale_lo)) : plain;
     }
 }
 
@@ -568,10 +569,10 @@ hipError_t welch_pair_residency(uint64_t n, int* per_cu)
 }
 
 hipError_t launch_spec_sum(const float* rows, float* acc, uint64_t nfreq, uint64_t nrows, bool first, float scale,
-                           hipStream_t s)
+                           hipStream_t s, float scale_lo)
 {
     hipLaunchKernelGGL(k_spec_sum, dim3(static_cast<unsigned>((nfreq + kSumBins - 1) / kSumBins)),
-                       dim3(kSumBins * kSumGroups), 0, s, rows, acc, nfreq, nrows, first ? 1 : 0, scale);
+                       dim3(kSumBins * kSumGroups), 0, s, rows, acc, nfreq, nrows, first ? 1 : 0, scale, scale_lo);
     return hipGetLastError();
 }
 
