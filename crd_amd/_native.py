@@ -24,6 +24,7 @@ FLAG_SEPARATE_PASSES = 4
 FLAG_CHIRP_Z = 8
 HINTS_NONE = 0x100
 HINT_TWO_PIPELINES = 0x20
+HINT_WHOLE = 0x80
 DCT2, DCT3, DST2, DST3 = 0, 1, 2, 3
 ND_TRANSPOSE_ALL = 1
 WINDOW_BOXCAR, WINDOW_HANN = 0, 1
@@ -46,6 +47,7 @@ class PlanInfo(ctypes.Structure):
         ("type", ctypes.c_int32),
         ("precision", ctypes.c_int32),
         ("algorithm", ctypes.c_int32),
+        ("whole", ctypes.c_uint32),
         ("complex_n", ctypes.c_uint64),
         ("n1", ctypes.c_uint64),
         ("n2", ctypes.c_uint64),

@@ -138,7 +138,7 @@ struct crdfft_plan_s
     DeviceBuffer thi, tlo;  // factored four-step twiddle
     DeviceBuffer tstep;     // column pass step table (e1 * n2 entries)
     DeviceBuffer tfull;     // column pass full twiddle table (n entries, small n only)
-    // whole-transform kernel of n = 2^15, 2^16 C2C and n = 2^16 R2C / C2R (untuned plans): W_256^e and the full
+    // whole-transform kernel of n = 2^15, 2^16 C2C and n = 2^16 R2C / C2R (PlanShape::whole): W_256^e and the full
     // four-step twiddle of 256 x complex_n / 256; whole_cus > 0 when the plan has it
     DeviceBuffer whole_roots, whole_full;
     uint32_t whole_cus = 0;
@@ -424,19 +424,10 @@ crdfft_status build_tables(crdfft_plan_s* p, hipStream_t s)
     return CRDFFT_OK;
 }
 
-// Of `count` transforms, how many the whole-transform kernel runs (the first ones; the four-step runs the rest). It takes
-// rounds of one transform per CU, so a partial round costs nearly a full one (256 CUs, n = 2^16 / 2^15: 60 / 26 us with
-// 96 transforms, 73 / 32 with 256) and the four-step about 0.37 / 0.21 us per transform. Alone, a partial round pays from
-// 176 / 128 transforms on (whole 66 / 27 us, four-step 67 / 28); behind full rounds it overlaps them and pays sooner: from
-// 96 (352 transforms: whole 126 / 60 us, split 126 / 64; 576, a rest of 64: 189 / 94, split 180 / 88), and behind four of
-// them from about 32 (1088, a rest of 64: 300 / 140, split 309 / 148).
-uint64_t whole_count(const crdfft_plan_s* p, uint64_t count)
+// Of `count` transforms of the plan, how many the whole-transform kernel runs.
+uint64_t whole_of(const crdfft_plan_s* p, uint64_t count)
 {
-    const uint64_t cus = p->whole_cus;
-    const uint64_t full = count / cus, rest = count % cus;
-    const uint64_t least = full == 0 ? (p->shape.complex_n == 65536 ? cus * 11 / 16 : cus / 2)
-                                     : (full < 4 ? cus * 3 / 8 : cus / 8);
-    return p->whole_always || rest >= least ? count : count - rest;
+    return p->whole_always ? count : crdfft::whole_count(p->shape.complex_n, p->whole_cus, count);
 }
 
 // The complex transform of the plan over `count` transforms (complex distances), on `s`.
@@ -488,7 +479,7 @@ crdfft_status run_complex(crdfft_plan_s* p, const cfloat* in, cfloat* out, uint6
                 (in == out ? idist == odist || count == 1
                            : in + (count - 1) * idist + cn <= out || out + (count - 1) * odist + cn <= in))
             {
-                const uint64_t whole = whole_count(p, count);
+                const uint64_t whole = whole_of(p, count);
                 if (whole > 0)
                 {
                     const crdfft::WholeArgs wa{in, out, p->whole_roots.as<cfloat>(), p->whole_full.as<cfloat>(),
@@ -687,7 +678,7 @@ crdfft_status run_whole_real(crdfft_plan_s* p, const cfloat* in, cfloat* out, ui
     {
         return CRDFFT_OK;
     }
-    *whole = whole_count(p, sh.batch);
+    *whole = whole_of(p, sh.batch);
     if (*whole > 0)
     {
         crdfft::WholeArgs wa{in, out, p->whole_roots.as<cfloat>(), p->whole_full.as<cfloat>(), *whole, idist, odist, 1.0f};
@@ -974,10 +965,7 @@ crdfft_status create_plan(crdfft_plan* plan, uint64_t n, uint64_t batch, uint64_
     p->odist = odist;
     p->flags = flags;
     (void)hipGetDevice(&p->device);
-    uint64_t whole_n2 = 0;
-    if (tuning == nullptr && shape.algorithm == CRDFFT_ALGO_FOUR_STEP && precision == CRDFFT_FP32 &&
-        crdfft::whole_kernel_n(shape.complex_n, &whole_n2) &&
-        (type == CRDFFT_C2C || (shape.complex_n == 32768 && (flags & CRDFFT_FLAG_SEPARATE_PASSES) == 0)))
+    if (shape.whole && (type == CRDFFT_C2C || (flags & CRDFFT_FLAG_SEPARATE_PASSES) == 0))
     {
         int cus = 0;
         if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, p->device) == hipSuccess && cus > 0)
@@ -1266,13 +1254,13 @@ crdfft_status plan_use_floor(crdfft_plan p)
     return CRDFFT_OK;
 }
 
-bool plan_uses_whole(crdfft_plan p) { return p->whole_cus > 0 && whole_count(p, p->shape.batch) > 0; }
+bool plan_uses_whole(crdfft_plan p) { return p->whole_cus > 0 && whole_of(p, p->shape.batch) > 0; }
 
 bool plan_uses_four_step(crdfft_plan p)
 {
     // (different distances: an in-place execute, which the whole-transform kernel cannot run)
     return p->whole_cus == 0 || (p->shape.type == CRDFFT_C2C && p->idist != p->odist) ||
-           whole_count(p, p->shape.batch) < p->shape.batch;
+           whole_of(p, p->shape.batch) < p->shape.batch;
 }
 
 crdfft_status plan_use_whole(crdfft_plan p)
@@ -1446,6 +1434,7 @@ crdfft_status crdfft_plan_get_info(crdfft_plan p, crdfft_plan_info* info)
         return CRDFFT_INVALID_ARGUMENT;
     }
     crdfft::shape_to_info(p->shape, info);
+    info->whole = p->whole_cus > 0 && !p->floor ? static_cast<uint32_t>(whole_of(p, p->shape.batch)) : 0u;
     info->check = p->check;
     info->table_bytes = p->tw_single.bytes + p->tw1.bytes + p->tw2.bytes + p->thi.bytes + p->tlo.bytes +
                         p->tstep.bytes + p->tfull.bytes + p->wreal.bytes + p->split_fwd[0].bytes + p->split_inv[0].bytes + p->split_tw[0].bytes +

@@ -80,6 +80,13 @@ namespace
 // A tuned hints field: CRDFFT_HINTS_NONE asks for none, other bits are kept where the algorithm has them.
 uint32_t tuning_hints(uint32_t h, uint32_t mask) { return (h & CRDFFT_HINTS_NONE) != 0 ? 0u : (h & mask); }
 
+// A tuning that names nothing: the planner's plan.
+bool is_default(const crdfft_tuning& t)
+{
+    return t.n1 == 0 && t.e == 0 && t.e1 == 0 && t.tile1 == 0 && t.e2 == 0 && t.tile2 == 0 && t.chunk == 0 && t.hints == 0 &&
+           t.algorithm == 0;
+}
+
 // Values per thread of the single kernel. C2C: the fastest per length in an autotune sweep over 2^22-point batches
 // on gfx950 (fewer values per thread keep more waves resident where a transform is short, and for 1024-4096 points
 // the extra LDS round trip of radix-8 stages costs less than the occupancy radix-16 gives up). R2C / C2R (n = the
@@ -189,6 +196,8 @@ crdfft_status choose_shape(uint64_t n, uint64_t batch, int32_t type, int32_t pre
     {
         return CRDFFT_INVALID_SIZE;
     }
+    // what the tuning says about cache hints and the schedule
+    const uint32_t asked = tuning != nullptr ? tuning->hints & ~CRDFFT_HINT_WHOLE : 0u;
     if (precision != CRDFFT_FP32)
     {
         // the split-precision MFMA passes run sequences of 256 (radix-16 stages) and 1024 points (radix-32): one
@@ -249,9 +258,9 @@ crdfft_status choose_shape(uint64_t n, uint64_t batch, int32_t type, int32_t pre
         {
             return CRDFFT_UNSUPPORTED;
         }
-        if (tuning != nullptr && tuning->hints != 0)
+        if (asked != 0)
         {
-            s.hints = tuning_hints(tuning->hints, 3u);
+            s.hints = tuning_hints(asked, 3u);
         }
     }
     else
@@ -319,9 +328,9 @@ crdfft_status choose_shape(uint64_t n, uint64_t batch, int32_t type, int32_t pre
             s.chunk = kDescribeCUs * per_cu;
             s.workspace_bytes = s.chunk * per + coop_ctl_words(s.chunk) * 4;
             s.hints = kDefaultFourStepHints;
-            if (tuning->hints != 0)
+            if (asked != 0)
             {
-                s.hints = tuning_hints(tuning->hints, 3u | kHintCoopSolo);
+                s.hints = tuning_hints(asked, 3u | kHintCoopSolo);
             }
             *out = s;
             return CRDFFT_OK;
@@ -358,9 +367,9 @@ crdfft_status choose_shape(uint64_t n, uint64_t batch, int32_t type, int32_t pre
             }
             s.workspace_bytes = s.chunk * per;
             s.hints = kDefaultFourStepHints;
-            if (tuning->hints != 0)
+            if (asked != 0)
             {
-                s.hints = tuning_hints(tuning->hints, 3u);
+                s.hints = tuning_hints(asked, 3u);
             }
             *out = s;
             return CRDFFT_OK;
@@ -381,9 +390,9 @@ crdfft_status choose_shape(uint64_t n, uint64_t batch, int32_t type, int32_t pre
         {
             s.hints |= kHintTwoPipes;
         }
-        if (tuning != nullptr && tuning->hints != 0)
+        if (asked != 0)
         {
-            s.hints = tuning_hints(tuning->hints, 11u | kHintTwoPipes);
+            s.hints = tuning_hints(asked, 11u | kHintTwoPipes);
         }
         // two pipelines keep two chunks in flight: each gets half the workspace budget. C2R, whose column pass reads
         // every bin twice (X[j] and X[h - j]), also runs half-size chunks: measured 3-11 % faster at n = 2^16..2^22;
@@ -404,9 +413,42 @@ crdfft_status choose_shape(uint64_t n, uint64_t batch, int32_t type, int32_t pre
         {
             return CRDFFT_UNSUPPORTED;
         }
+        uint64_t whole_n2 = 0;
+        s.whole = whole_kernel_n(cn, &whole_n2) && (type == CRDFFT_C2C || cn == 32768) &&
+                  (tuning == nullptr || (tuning->hints & CRDFFT_HINT_WHOLE) != 0 || is_default(*tuning));
     }
     *out = s;
     return CRDFFT_OK;
+}
+
+// Of `count` transforms, how many the whole-transform kernel runs (the first ones; the four-step runs the rest). It takes
+// rounds of one transform per CU, so a partial round costs nearly a full one (256 CUs, n = 2^16 / 2^15: 60 / 26 us with
+// 96 transforms, 73 / 32 with 256) and the four-step about 0.37 / 0.21 us per transform. Alone, a partial round pays from
+// 176 / 128 transforms on (whole 66 / 27 us, four-step 67 / 28); behind full rounds it overlaps them and pays sooner: from
+// 96 (352 transforms: whole 126 / 60 us, split 126 / 64; 576, a rest of 64: 189 / 94, split 180 / 88), and behind four of
+// them from about 32 (1088, a rest of 64: 300 / 140, split 309 / 148).
+uint64_t whole_count(uint64_t complex_n, uint64_t cus, uint64_t count)
+{
+    const uint64_t full = count / cus, rest = count % cus;
+    const uint64_t least = full == 0 ? (complex_n == 65536 ? cus * 11 / 16 : cus / 2)
+                                     : (full < 4 ? cus * 3 / 8 : cus / 8);
+    return rest >= least ? count : count - rest;
+}
+
+crdfft_tuning tuning_of(const crdfft_plan_info& info)
+{
+    crdfft_tuning t{};
+    t.n1 = info.n1;
+    t.e = info.e;
+    t.e1 = info.e1;
+    t.tile1 = info.tile1;
+    t.e2 = info.e2;
+    t.tile2 = info.tile2;
+    t.chunk = info.chunk;
+    t.hints = info.hints == 0 ? CRDFFT_HINTS_NONE : info.hints; // a tuning's 0 would mean the planner's default
+    t.hints |= info.whole > 0 ? CRDFFT_HINT_WHOLE : 0u;
+    t.algorithm = info.algorithm;
+    return t;
 }
 
 void shape_to_info(const PlanShape& s, crdfft_plan_info* info)
@@ -428,6 +470,7 @@ void shape_to_info(const PlanShape& s, crdfft_plan_info* info)
     info->chunk = s.chunk;
     info->workspace_bytes = s.workspace_bytes;
     info->hints = s.hints;
+    info->whole = s.whole ? static_cast<uint32_t>(whole_count(s.complex_n, kDescribeCUs, s.batch)) : 0u;
 }
 
 } // namespace crdfft

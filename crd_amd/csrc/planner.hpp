@@ -30,6 +30,7 @@ struct PlanShape
     uint64_t workspace_bytes = 0;
     uint32_t hints = 0; // kHintNtLoad | kHintNtStore
     int32_t threads = 0; // fused four-step: workgroup size (tile1 columns, tile2 rows per tile)
+    bool whole = false;  // four-step: whole transforms on one CU each for whole_count() of the batch
 };
 
 // The largest complex length one LDS-resident kernel runs.
@@ -55,7 +56,7 @@ constexpr uint64_t kFusedMax = uint64_t{1} << 17;
 // Workgroup size of the fused four-step unless tuned: 512 threads (two workgroups per CU hide each other's memory
 // waits).
 constexpr int kFusedThreads = 512;
-// CUs assumed by crdfft_plan_describe for the fused slot count (plan creation asks the device).
+// CUs assumed by crdfft_plan_describe for the fused slot count and the whole transforms (plan creation asks the device).
 constexpr uint64_t kDescribeCUs = 256;
 // Up to this length the column pass reads its twiddle W_N^{n2 k1} from one full table (n entries, at most 2 MiB,
 // L2-resident): one load and one complex multiply per value instead of two multiplies.
@@ -66,6 +67,12 @@ uint32_t log2_exact(uint64_t n);
 
 crdfft_status choose_shape(uint64_t n, uint64_t batch, int32_t type, int32_t precision, const crdfft_tuning* tuning,
                            PlanShape* out);
+// Of `count` transforms of a `whole` shape of complex_n points, how many (the first ones) the whole-transform kernel runs
+// on a device of `cus` CUs.
+uint64_t whole_count(uint64_t complex_n, uint64_t cus, uint64_t count);
+// A tuning that gives a plan of this shape back, for the same batch.
+crdfft_tuning tuning_of(const crdfft_plan_info& info);
+// info.whole for a device of kDescribeCUs CUs (a plan counts its own device's).
 void shape_to_info(const PlanShape& s, crdfft_plan_info* info);
 
 // Values per thread and columns per workgroup of the element-major kernel for n (e depends on n only).
@@ -88,8 +95,8 @@ constexpr uint32_t kCoopSpinLimit = 1u << 18;
 crdfft_status plan_use_floor(crdfft_plan p);
 bool plan_on_floor(crdfft_plan p);
 
-// Plans of n = 2^15 and 2^16 (C2C, untuned): whether their batch runs on the whole-transform kernel, on the four-step
-// (a batch with a small last round runs on both), and switching a self-check's one-transform plan onto the former.
+// Plans with PlanShape::whole: whether their batch runs on the whole-transform kernel, on the four-step (a batch with a
+// small last round runs on both), and switching a self-check's one-transform plan onto the former.
 bool plan_uses_whole(crdfft_plan p);
 bool plan_uses_four_step(crdfft_plan p);
 crdfft_status plan_use_whole(crdfft_plan p);

@@ -22,22 +22,7 @@ namespace
 bool same_shape(const crdfft::PlanShape& a, const crdfft::PlanShape& b)
 {
     return a.algorithm == b.algorithm && a.n1 == b.n1 && a.e == b.e && a.e1 == b.e1 && a.tile1 == b.tile1 &&
-           a.e2 == b.e2 && a.tile2 == b.tile2 && a.chunk == b.chunk && a.hints == b.hints && a.threads == b.threads;
-}
-
-crdfft_tuning tuning_of(const crdfft::PlanShape& s)
-{
-    crdfft_tuning t{};
-    t.n1 = s.n1;
-    t.e = s.e;
-    t.e1 = s.e1;
-    t.tile1 = s.tile1;
-    t.e2 = s.e2;
-    t.tile2 = s.tile2;
-    t.chunk = s.chunk;
-    t.hints = s.hints == 0 ? CRDFFT_HINTS_NONE : s.hints; // a tuning's 0 would mean the planner's default
-    t.algorithm = s.algorithm;
-    return t;
+           a.e2 == b.e2 && a.tile2 == b.tile2 && a.chunk == b.chunk && a.hints == b.hints && a.threads == b.threads && a.whole == b.whole;
 }
 
 std::vector<crdfft_tuning> enumerate(uint64_t n, uint64_t batch, int32_t type)
@@ -50,6 +35,9 @@ std::vector<crdfft_tuning> enumerate(uint64_t n, uint64_t batch, int32_t type)
         {
             return;
         }
+        crdfft_plan_info info;
+        crdfft::shape_to_info(s, &info);
+        s.whole = info.whole > 0; // no whole transforms at this batch: the two passes
         for (const crdfft::PlanShape& q : shapes)
         {
             if (same_shape(q, s))
@@ -58,7 +46,7 @@ std::vector<crdfft_tuning> enumerate(uint64_t n, uint64_t batch, int32_t type)
             }
         }
         shapes.push_back(s);
-        out.push_back(tuning_of(s));
+        out.push_back(crdfft::tuning_of(info));
     };
     add(nullptr); // candidate 0: the planner's default
     crdfft::PlanShape def;
@@ -275,15 +263,7 @@ crdfft_status crdfft_time_plan(uint64_t n, uint64_t batch, int32_t type, const c
     record->precision = CRDFFT_FP32;
     record->ndim = 1;
     record->dims[0] = n;
-    record->tuning.n1 = info.n1;
-    record->tuning.e = info.e;
-    record->tuning.e1 = info.e1;
-    record->tuning.tile1 = info.tile1;
-    record->tuning.e2 = info.e2;
-    record->tuning.tile2 = info.tile2;
-    record->tuning.chunk = info.chunk;
-    record->tuning.hints = info.hints == 0 ? CRDFFT_HINTS_NONE : info.hints; // replayable: 0 means the default
-    record->tuning.algorithm = info.algorithm;
+    record->tuning = crdfft::tuning_of(info);
     record->algorithm = info.algorithm;
     record->ms = ms[ms.size() / 2];
     return CRDFFT_OK;
@@ -387,7 +367,11 @@ crdfft_status crdfft_plan_features(const crdfft_plan_record* records, uint64_t c
         f[28] = r.ndim >= 2 ? log2f_safe(static_cast<double>(r.dims[0])) / 12.0f : 0.0f;
         f[29] = r.ndim >= 3 ? log2f_safe(static_cast<double>(r.dims[1])) / 12.0f : 0.0f;
         f[30] = r.algorithm == CRDFFT_ALGO_FOUR_STEP ? 1.0f : 0.0f;
-        f[31] = r.algorithm == CRDFFT_ALGO_FUSED ? 1.0f : (r.algorithm == CRDFFT_ALGO_COOP ? 0.5f : 0.0f);
+        // the one-launch forms of the longer lengths
+        f[31] = r.algorithm == CRDFFT_ALGO_FUSED          ? 1.0f
+                : r.algorithm == CRDFFT_ALGO_COOP         ? 0.5f
+                : (r.tuning.hints & CRDFFT_HINT_WHOLE) != 0 ? 0.75f
+                                                            : 0.0f;
     }
     return CRDFFT_OK;
 }

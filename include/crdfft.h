@@ -82,9 +82,10 @@ typedef enum crdfft_algorithm
     CRDFFT_ALGO_COPY = 0,       /* n == 1 */
     CRDFFT_ALGO_SINGLE = 1,     /* one LDS-staged kernel per transform (n <= 16384) */
     CRDFFT_ALGO_FOUR_STEP = 2,  /* n = n1*n2: column pass with twiddle, row pass with transposed store. Plans of 2^15 and
-                                   2^16 complex points (C2C; R2C / C2R of 2^16) without tuning run both steps of a
-                                   transform on one CU in one launch for as much of the batch as fills the device
-                                   (crdfft_phase_times: phase 0), the two passes for the rest */
+                                   2^16 complex points (C2C; R2C / C2R of 2^16) without tuning, or tuned with
+                                   CRDFFT_HINT_WHOLE, run both steps of a transform on one CU in one launch for as much
+                                   of the batch as fills the device (crdfft_plan_info.whole; crdfft_phase_times: phase
+                                   0), the two passes for the rest */
     CRDFFT_ALGO_REFERENCE = 3,  /* the radix-2 reference only */
     CRDFFT_ALGO_BLUESTEIN = 4,  /* chirp-z over a power-of-two plan of m >= 2n-1 (any n) */
     CRDFFT_ALGO_FUSED = 5,      /* n = n1*n2 <= 2^17: both four-step passes of a transform in one workgroup of a
@@ -113,6 +114,8 @@ typedef struct crdfft_plan_info
     int32_t type;         /* crdfft_type */
     int32_t precision;    /* crdfft_precision */
     int32_t algorithm;    /* crdfft_algorithm of the complex transform that runs */
+    uint32_t whole;       /* four-step: how many of the batch, the first ones, run as whole transforms on one CU each
+                             (out of place, or in place with idist == odist), the others in two passes */
     uint64_t complex_n;   /* length of the complex transform (n/2 for R2C/C2R) */
     uint64_t n1, n2;      /* four-step split (0 for single) */
     int32_t e;            /* values per thread of the single/row kernel */
@@ -149,6 +152,11 @@ typedef enum crdfft_check_status
  * and at least two chunks; the first execute on a caller stream creates that stream's pipeline, and an execute
  * captured into a graph before the pipeline exists records both halves on the captured stream instead. */
 #define CRDFFT_HINT_TWO_PIPELINES 0x20u
+/* crdfft_tuning.hints, four-step plans of 2^15 and 2^16 complex points (C2C; R2C / C2R of 2^16 without
+ * CRDFFT_FLAG_SEPARATE_PASSES): whole transforms on one CU each for as much of the batch as fills the device, as in a plan
+ * without tuning. The other fields, and the other hints where there are any, tune the two passes of the rest. Without this
+ * bit a tuning that names anything runs two passes throughout; a tuning of zeros is the planner's plan. */
+#define CRDFFT_HINT_WHOLE 0x80u
 typedef struct crdfft_tuning
 {
     uint64_t n1;          /* four-step split */

@@ -118,6 +118,45 @@ def test_planner_four_step_schedules():
     assert info.hints == 3 | two and info.chunk == 4
 
 
+def _describe_tuned(n, batch, type, tuning):
+    import ctypes
+
+    from crd_amd import _native as N
+
+    info = N.PlanInfo()
+    N.check(N.lib().crdfft_plan_describe_tuned(n, batch, type, N.FP32, ctypes.byref(tuning), ctypes.byref(info)))
+    return info
+
+
+def test_whole_transforms_in_tunings():
+    """The planner's plan of 2^15 / 2^16 complex points runs whole transforms (crdfft_plan_info.whole): candidate 0 of the
+    tuner is that plan and says so, a tuning of zeros is that plan, and one that names a knob is not unless it asks."""
+    import crd_amd
+    from crd_amd import _native as N
+    from crd_amd import costmodel
+
+    for n, batch, name, type, whole in ((1 << 16, 512, "c2c", N.C2C, 512), (1 << 16, 300, "c2c", N.C2C, 256),
+                                        (1 << 15, 128, "c2c", N.C2C, 128), (1 << 16, 256, "r2c", N.R2C, 256),
+                                        (1 << 16, 1100, "c2r", N.C2R, 1100), (1 << 16, 64, "c2c", N.C2C, 0),
+                                        (1 << 15, 512, "r2c", N.R2C, 0), (1 << 17, 512, "c2c", N.C2C, 0)):
+        plain = crd_amd.describe(n, batch, name)
+        assert plain["whole"] == whole, (n, batch, name)
+        cands = costmodel.candidates(n, batch, name)
+        assert bool(cands[0].hints & N.HINT_WHOLE) == (whole > 0)
+        assert not any(c.hints & N.HINT_WHOLE for c in cands[1:])
+        for same in (cands[0], N.Tuning(), N.Tuning(hints=N.HINT_WHOLE)):
+            assert _describe_tuned(n, batch, type, same).as_dict() == plain, (n, batch, name)
+        settings = [tuple(getattr(c, f) for f, _ in N.Tuning._fields_) for c in cands]
+        assert len(set(settings)) == len(settings)
+        if plain["algorithm"] == 2:
+            two = N.Tuning(chunk=plain["chunk"])
+            assert _describe_tuned(n, batch, type, two).whole == 0
+            two.hints = N.HINT_WHOLE
+            assert _describe_tuned(n, batch, type, two).as_dict() == plain
+    info = _describe_tuned(1 << 16, 512, N.C2C, N.Tuning(algorithm=N.ALGO_FUSED, hints=N.HINT_WHOLE))
+    assert (info.algorithm, info.whole) == (N.ALGO_FUSED, 0)
+
+
 def test_tuning_hints_none_is_explicit():
     """CRDFFT_HINTS_NONE asks for plain loads and stores; 0 keeps the planner's default."""
     import crd_amd

@@ -136,3 +136,37 @@ def test_rerun_of_the_real_forms_is_bit_identical(gpu):
         out.append((spec.download((batch, h + 1), np.complex64), back.download((batch, n), np.float32)))
     for a, b in zip(*out):
         assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
+@pytest.mark.parametrize("n,batch,type", [(1 << 16, 512, "c2c"), (1 << 15, 300, "c2c"), (1 << 16, 512, "r2c"),
+                                          (1 << 16, 300, "c2r")])
+def test_tuning_reaches_the_planners_plan(gpu, n, batch, type):
+    """Candidate 0 of the tuner, and the tuning of a record of the untuned plan, launch what an untuned plan launches."""
+    import ctypes
+
+    from crd_amd import _native as N
+    from crd_amd import costmodel
+
+    code = {"c2c": N.C2C, "r2c": N.R2C, "c2r": N.C2R}[type]
+    direction = gpu.INVERSE if type == "c2r" else gpu.FORWARD
+    src, dst = gpu.DeviceBuffer(8 * (n + 2) * batch), gpu.DeviceBuffer(8 * (n + 2) * batch)
+    src.fill(0)
+
+    def launches(tuning):
+        plan = gpu.FftPlan(n, batch, type, tuning=tuning)
+        assert plan.info()["check"] == N.CHECK_PASSED
+        acc = plan.execute_profiled(src, dst, direction)
+        return [acc.launches[i] for i in range(4)], [acc.points[i] for i in range(4)], plan.info()["whole"]
+
+    plain = launches(None)
+    assert plain[2] > 0
+    rec = N.PlanRecord()
+    N.check(N.lib().crdfft_time_plan(n, batch, code, None, 3, ctypes.byref(rec)))
+    for t in (costmodel.candidates(n, batch, type)[0], rec.tuning):
+        assert launches({f: getattr(t, f) for f, _ in N.Tuning._fields_}) == plain
+    best = N.Tuning()
+    N.check(N.lib().crdfft_autotune_plan(n, batch, code, 5, ctypes.byref(best), None, 0, None))
+    N.check(N.lib().crdfft_time_plan(n, batch, code, ctypes.byref(best), 9, ctypes.byref(rec)))
+    tuned = rec.ms
+    N.check(N.lib().crdfft_time_plan(n, batch, code, None, 9, ctypes.byref(rec)))
+    assert tuned <= 1.15 * rec.ms  # the two passes take 1.2-1.9x here
