@@ -1256,13 +1256,6 @@ crdfft_status plan_use_floor(crdfft_plan p)
 
 bool plan_uses_whole(crdfft_plan p) { return p->whole_cus > 0 && whole_of(p, p->shape.batch) > 0; }
 
-bool plan_uses_four_step(crdfft_plan p)
-{
-    // (different distances: an in-place execute, which the whole-transform kernel cannot run)
-    return p->whole_cus == 0 || (p->shape.type == CRDFFT_C2C && p->idist != p->odist) ||
-           whole_of(p, p->shape.batch) < p->shape.batch;
-}
-
 crdfft_status plan_use_whole(crdfft_plan p)
 {
     p->whole_cus = 1;

@@ -95,10 +95,9 @@ constexpr uint32_t kCoopSpinLimit = 1u << 18;
 crdfft_status plan_use_floor(crdfft_plan p);
 bool plan_on_floor(crdfft_plan p);
 
-// Plans with PlanShape::whole: whether their batch runs on the whole-transform kernel, on the four-step (a batch with a
-// small last round runs on both), and switching a self-check's one-transform plan onto the former.
+// Plans with PlanShape::whole: whether any of their batch runs on the whole-transform kernel, and switching a self-check's
+// one-transform plan onto it.
 bool plan_uses_whole(crdfft_plan p);
-bool plan_uses_four_step(crdfft_plan p);
 crdfft_status plan_use_whole(crdfft_plan p);
 
 } // namespace crdfft

@@ -9,7 +9,8 @@
 // A failing check returns CRDFFT_SELF_CHECK_FAILED; plan creation then demotes the plan to its floor (the radix-2
 // reference kernels) and checks again (crdfft_check_status). CRDFFT_FAULT_SELF_CHECK in the environment corrupts one
 // output value before the comparison, the host fault seam (reference crd/core/fault_seam.hpp:139) that lets a test
-// force either path: "1" for the selected kernels only, "2" for every check.
+// force either path: "1" for the selected kernels only, "2" for every check, "3" for the two passes of plans that also run
+// whole transforms.
 #include <cmath>
 #include <complex>
 #include <cstdlib>
@@ -41,15 +42,15 @@ struct DevBuf
 };
 
 // The fault seam: "1" fails the check of a plan's selected kernels (so it demotes to its floor), "2" fails every
-// check (the floor's too).
-bool fault_forced(crdfft_plan plan)
+// check (the floor's too), "3" only that of the two passes of a plan that also runs whole transforms (`beside_whole`).
+bool fault_forced(crdfft_plan plan, bool beside_whole)
 {
     const char* v = std::getenv("CRDFFT_FAULT_SELF_CHECK");
     if (v == nullptr)
     {
         return false;
     }
-    return v[0] == '2' || (v[0] == '1' && !crdfft::plan_on_floor(plan));
+    return v[0] == '2' || (v[0] == '1' && !crdfft::plan_on_floor(plan)) || (v[0] == '3' && beside_whole);
 }
 
 // The single-transform plan the check runs: the same kernels as `plan`, on its floor when the plan is.
@@ -119,7 +120,9 @@ extern "C" crdfft_status crdfft_self_check(crdfft_plan plan)
     const uint64_t n = info.n;
     const double lg = std::max(1.0, std::log2(static_cast<double>(n)));
     const double tol = 2e-6 * lg;
-    const bool fault = fault_forced(plan);
+    // A plan that runs whole transforms also runs its two passes, whatever its batch: where the rows of input and output lie
+    // between each other, or in place at different distances. Both forms are checked.
+    const bool whole = !crdfft::plan_on_floor(plan) && crdfft::plan_uses_whole(plan);
 
     if (info.type == CRDFFT_C2C)
     {
@@ -141,12 +144,11 @@ extern "C" crdfft_status crdfft_self_check(crdfft_plan plan)
             return st;
         }
         crdfft_status result = CRDFFT_OK;
-        // both directions on the four-step or single kernel, then on the whole-transform kernel, as the plan uses them
-        const bool whole = !crdfft::plan_on_floor(plan) && crdfft::plan_uses_whole(plan);
-        const int first = whole && !crdfft::plan_uses_four_step(plan) ? 2 : 0;
-        for (int form = first; form < (whole ? 4 : 2) && result == CRDFFT_OK; ++form)
+        // both directions on the four-step or single kernel, then on the whole-transform kernel
+        for (int form = 0; form < (whole ? 4 : 2) && result == CRDFFT_OK; ++form)
         {
             const int dir = form & 1;
+            const bool fault = fault_forced(plan, whole && form < 2);
             if (form == 2)
             {
                 result = crdfft::plan_use_whole(one);
@@ -251,11 +253,10 @@ extern "C" crdfft_status crdfft_self_check(crdfft_plan plan)
         return st;
     }
     crdfft_status result = CRDFFT_OK;
-    // on the four-step or single kernel, then on the whole-transform kernel, as the plan uses them
-    const bool whole = !crdfft::plan_on_floor(plan) && crdfft::plan_uses_whole(plan);
-    const int first = whole && !crdfft::plan_uses_four_step(plan) ? 1 : 0;
-    for (int form = first; form < (whole ? 2 : 1) && result == CRDFFT_OK; ++form)
+    // on the four-step or single kernel, then on the whole-transform kernel
+    for (int form = 0; form < (whole ? 2 : 1) && result == CRDFFT_OK; ++form)
     {
+        const bool fault = fault_forced(plan, whole && form == 0);
         if (form == 1)
         {
             result = crdfft::plan_use_whole(one);

@@ -136,7 +136,7 @@ typedef struct crdfft_plan_info
  * there: DEMOTED. When the floor fails too, creation returns CRDFFT_SELF_CHECK_FAILED (the reference runs its
  * portable table then; a device whose simplest kernels misexecute has nothing safer to offer). Fault seam:
  * CRDFFT_FAULT_SELF_CHECK=1 in the environment fails the selected kernels' check (the plan demotes), =2 fails
- * every check. Element-major batches (crdfft_execute_batched) keep their own kernels. */
+ * every check, =3 fails that of the two passes of a plan that also runs whole transforms. Element-major batches (crdfft_execute_batched) keep their own kernels. */
 typedef enum crdfft_check_status
 {
     CRDFFT_CHECK_NOT_RUN = 0, /* CRDFFT_FLAG_NO_SELF_CHECK, or a plan kind the check does not cover */

@@ -170,3 +170,37 @@ def test_tuning_reaches_the_planners_plan(gpu, n, batch, type):
     tuned = rec.ms
     N.check(N.lib().crdfft_time_plan(n, batch, code, None, 9, ctypes.byref(rec)))
     assert tuned <= 1.15 * rec.ms  # the two passes take 1.2-1.9x here
+
+
+@pytest.mark.parametrize("n,batch,type", [(1 << 15, 256, "c2c"), (1 << 16, 256, "c2c"), (1 << 16, 256, "r2c"),
+                                          (1 << 16, 256, "c2r")])
+def test_both_forms_are_checked(gpu, n, batch, type):
+    """A batch of whole transforms alone runs two passes where its buffers ask for it (below), so a plan whose two passes
+    fail their check is demoted too."""
+    import os
+
+    from crd_amd import _native as N
+
+    os.environ["CRDFFT_FAULT_SELF_CHECK"] = "3"
+    try:
+        plan = gpu.FftPlan(n, batch, type)
+    finally:
+        del os.environ["CRDFFT_FAULT_SELF_CHECK"]
+    assert plan.info()["check"] == N.CHECK_DEMOTED and plan.info()["whole"] == 0
+    assert plan.self_check() == N.OK
+    plan = gpu.FftPlan(n, batch, type)
+    assert plan.info()["check"] == N.CHECK_PASSED and plan.info()["whole"] == batch
+
+
+def test_rows_between_the_rows_of_the_input(gpu, po):
+    """Input and output rows in turn in one allocation: disjoint, but their ranges overlap, so two passes run them."""
+    n, batch = 1 << 15, 256
+    x = _input(np.random.default_rng(9), batch, n, 2 * n)
+    buf = gpu.DeviceBuffer.from_array(x)
+    plan = gpu.FftPlan(n, batch, idist=2 * n, odist=2 * n)
+    acc = plan.execute_profiled(buf.address, buf.address + 8 * n, gpu.FORWARD)
+    assert acc.launches[1] > 0
+    y = buf.download((batch, 2 * n), np.complex64)
+    assert np.array_equal(y[:, :n].view(np.uint32), x[:, :n].view(np.uint32))
+    rows = [0, 1, 100, batch - 1]
+    assert po.rel_l2(y[rows, n:], po.fft64_of_f32(np.ascontiguousarray(x[rows, :n]))) <= bound(n)
