@@ -177,7 +177,8 @@ __global__ __launch_bounds__((SpecCfg<H, E>::threads)) void k_spec(SpecArgs a)
                                  : (T >= 16 ? view.get_at(pad16(T - i), T * (E - 1 - m)) : view.get(H - k));
             const cf e = {(zk.x + zh.x) * 0.5f, (zk.y - zh.y) * 0.5f};
             const cf o = {(zk.y + zh.y) * 0.5f, (zh.x - zk.x) * 0.5f};
-            const cf xk = cadd(e, cmul(o, wk[k]));
+            // X[0] without its products: they are exact, but infinity times the zero parts would be NaN
+            const cf xk = m == 0 && k == 0 ? cf{zk.x + zk.y, 0.0f} : cadd(e, cmul(o, wk[k]));
             // k == 0 also yields the Nyquist bin: W_N^H = -1, X[H] = Re Z0 - Im Z0 (read only where k == 0)
             const cf xn = {zk.x - zk.y, 0.0f};
             if constexpr (MODE == 0)

@@ -727,6 +727,12 @@ template <int NT, bool INV, int KIND> __global__ __launch_bounds__(512) void k_w
             {
                 cf xk, xh;
                 mirror_pair(z[r], p[r], cmul(wk, wk2[r]), xk, xh);
+                if (j == 0 && r == 0)
+                {
+                    // X[0] and X[h] without their products (exact, but for an infinity times the zero parts)
+                    xk = tid == 0 ? cf{z[0].x + z[0].y, 0.0f} : xk;
+                    xh = tid == 0 ? cf{z[0].x - z[0].y, 0.0f} : xh;
+                }
                 const uint32_t step = 65536u * static_cast<uint32_t>(r), step_h = 65536u * static_cast<uint32_t>(3 - r);
                 if (j == 0)
                 {
