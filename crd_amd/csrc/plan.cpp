@@ -1431,7 +1431,8 @@ crdfft_status crdfft_plan_get_info(crdfft_plan p, crdfft_plan_info* info)
     info->check = p->check;
     info->table_bytes = p->tw_single.bytes + p->tw1.bytes + p->tw2.bytes + p->thi.bytes + p->tlo.bytes +
                         p->tstep.bytes + p->tfull.bytes + p->wreal.bytes + p->split_fwd[0].bytes + p->split_inv[0].bytes + p->split_tw[0].bytes +
-                        p->split_fwd[1].bytes + p->split_inv[1].bytes + p->split_tw[1].bytes + p->split_tcm.bytes;
+                        p->split_fwd[1].bytes + p->split_inv[1].bytes + p->split_tw[1].bytes + p->split_tcm.bytes +
+                        p->whole_roots.bytes + p->whole_full.bytes;
     return CRDFFT_OK;
 }
 

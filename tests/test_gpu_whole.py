@@ -204,3 +204,11 @@ def test_rows_between_the_rows_of_the_input(gpu, po):
     assert np.array_equal(y[:, :n].view(np.uint32), x[:, :n].view(np.uint32))
     rows = [0, 1, 100, batch - 1]
     assert po.rel_l2(y[rows, n:], po.fft64_of_f32(np.ascontiguousarray(x[rows, :n]))) <= bound(n)
+
+
+@pytest.mark.parametrize("n,type", [(1 << 15, "c2c"), (1 << 16, "c2c"), (1 << 16, "r2c")])
+def test_table_bytes_count_the_whole_transforms_tables(gpu, n, type):
+    plan = gpu.FftPlan(n, 256, type)
+    two = gpu.FftPlan(n, 256, type, tuning={"chunk": plan.info()["chunk"]})
+    points = plan.info()["complex_n"] + 256  # the four-step twiddle of 256 x n2 and W_256
+    assert plan.info()["table_bytes"] == two.info()["table_bytes"] + 8 * points
