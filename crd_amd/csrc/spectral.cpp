@@ -116,20 +116,22 @@ crdfft_status run(crdfft_spectral_plan p, const float* x, uint64_t len, int mode
         const uint64_t wgs = std::min<uint64_t>((pairs + p->ppg - 1) / p->ppg, p->pair_wgs);
         a.out = partial;
         a.tw = p->pair_tw.as<crdfft::cfloat>();
-        // the frames are scaled by a power of two near 1 / (fs sum w^2), exactly, and the row sum by the rest over the frame
-        // count in two parts: rounded scales would be one error common to all bins
+        // The window carries a power of two whose square is at most 1 / (fs sum w^2), exactly, and the row sum is scaled by the
+        // rest over the frame count in two parts: rounded scales would be one error common to all bins. A bin of a pair can
+        // be |A| + |B|, so its square unscaled would leave the range at half the amplitude of a single frame's; scaled it is
+        // at most twice the scaled squares of A and B, which the sum adds up in any case (from a scale of 1 on as it is).
         const double scale = 1.0 / (fs * p->winsum2);
-        double rest = 1.0 / static_cast<double>(frames);
-        const double pow2 = std::exp2(std::round(std::log2(scale)));
-        if (pow2 > 1e-36 && pow2 < 1e36)
+        double fold = 1.0;
+        if (scale < 1.0)
         {
-            a.scale = static_cast<float>(pow2);
-            rest = scale / pow2 / static_cast<double>(frames);
+            fold = std::exp2(std::max(std::floor(0.5 * std::log2(scale)), -60.0));
         }
+        a.scale = static_cast<float>(fold);
+        const double rest = scale / (fold * fold) / static_cast<double>(frames);
         const float rest_hi = static_cast<float>(rest);
+        const float rest_lo = std::isfinite(rest_hi) ? static_cast<float>(rest - static_cast<double>(rest_hi)) : 0.0f;
         SPEC_TRY(crdfft::launch_welch_pairs(p->nperseg, a, wgs, s));
-        SPEC_TRY(crdfft::launch_spec_sum(partial, psd, nfreq, wgs, true, rest_hi, s,
-                                         static_cast<float>(rest - static_cast<double>(rest_hi))));
+        SPEC_TRY(crdfft::launch_spec_sum(partial, psd, nfreq, wgs, true, rest_hi, s, rest_lo));
         return CRDFFT_OK;
     }
     if (p->h <= static_cast<uint64_t>(crdfft::kSpecWelchMaxH))

@@ -18,7 +18,7 @@ struct SpecArgs
     void* out;           // complex rows, density rows, or partial rows (by mode)
     uint64_t frames;
     uint64_t hop;
-    float scale;         // 1 / (fs * sum w^2) of the density modes
+    float scale;         // 1 / (fs * sum w^2) of the density modes; pairs of frames: the window's power of two
     int32_t detrend;     // subtract each frame's mean
     uint64_t ostride;    // output row pitch in elements (complex for mode 0, float for mode 1), >= H + 1
 };

@@ -239,7 +239,7 @@ __global__ __launch_bounds__((SpecCfg<H, E>::threads)) void k_spec(SpecArgs a)
 
 // k_welch<N, E>: the Welch sum over pairs of frames. Frames 2 p and 2 p + 1 are the real and imaginary parts of one
 // N-point transform Z, and |A[k]|^2 + |B[k]|^2 = (|Z[k]|^2 + |Z[N-k]|^2) / 2, so nothing has to be told apart per
-// frame: a lane group of T = N/E threads adds scale |Z[k]|^2 of its pairs g, g + G, ... to its E slots, folds k onto
+// frame: a lane group of T = N/E threads adds |Z[k]|^2 of its pairs g, g + G, ... to its E slots, folds k onto
 // N - k through LDS once at the end and the workgroup writes one partial row of N/2 + 1 densities. Per frame that is half an N-point
 // transform (12 levels of 4096 points for two frames) in place of a half-length one, a recombine and its LDS exchange.
 // Bound by the vector unit (about 900 instructions a thread and pair at N = 4096, E = 16; floor by bytes 44 us). Measured,
@@ -297,7 +297,7 @@ __global__ __launch_bounds__((WelchCfg<N, E>::threads)) void k_welch(SpecArgs a)
 #pragma unroll
     for (int m = 0; m < E; ++m)
     {
-        win[m] = a.window != nullptr ? bld32<0>(wr, o4, 4u * T * m) : 1.0f;
+        win[m] = (a.window != nullptr ? bld32<0>(wr, o4, 4u * T * m) : 1.0f) * a.scale; // a power of two
     }
 #pragma unroll 1
     for (uint64_t it = 0; it < iters; ++it)
@@ -342,21 +342,18 @@ __global__ __launch_bounds__((WelchCfg<N, E>::threads)) void k_welch(SpecArgs a)
                 v[m] = csub(v[m], mean);
             }
         }
-        if (a.window != nullptr)
-        {
 #pragma unroll
-            for (int m = 0; m < E; ++m)
-            {
-                v[m].x *= win[m];
-                v[m].y *= win[m];
-            }
+        for (int m = 0; m < E; ++m)
+        {
+            v[m].x *= win[m];
+            v[m].y *= win[m];
         }
         fft_core<N, E, false, 1>(v, i, view, reinterpret_cast<const cf*>(a.tw));
         // an idle lane group or half of a pair: the samples are zeros, less a mean of zero
 #pragma unroll
         for (int m = 0; m < E; ++m)
         {
-            acc[m] += a.scale * (v[m].x * v[m].x + v[m].y * v[m].y);
+            acc[m] += v[m].x * v[m].x + v[m].y * v[m].y;
         }
     }
     // the lane groups' sums in group order, k folded onto N - k: P[k] = S[k] + S[N - k] (the one-sided doubling of the

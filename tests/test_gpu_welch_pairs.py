@@ -1,7 +1,7 @@
 """Welch over pairs of frames (two frames per complex transform) at the frame counts where it takes over from single frames
 (512 up to 256 samples a frame, 1024 above), odd counts (half a pair), odd hops (frames on any 4-byte boundary) and both
 window / detrend settings, against the oracle's FP64 restatement: rel-L2 <= 2e-6 log2(nperseg), the bar of the spectral
-tests. A NaN sample reaches every bin, a zero signal gives zeros, reruns are bit-identical."""
+tests, also where a pair's squares would leave the range unscaled. A NaN sample reaches every bin, a zero signal gives zeros, reruns are bit-identical."""
 import numpy as np
 import pytest
 
@@ -53,3 +53,21 @@ def test_nan_and_zeros(gpu, nperseg):
     assert not np.any(_welch(gpu, x, nperseg, nperseg // 2, "hann", True)[1])
     x[nperseg * 700 + 3] = np.nan
     assert np.all(np.isnan(_welch(gpu, x, nperseg, nperseg // 2, "hann", True)[1]))
+
+
+@pytest.mark.parametrize("nperseg,window,fs", [(64, "hann", 48000.0), (512, "boxcar", 48000.0), (512, "hann", 1e-3),
+                                               (4096, "hann", 1.0)])
+def test_amplitudes_near_the_range(gpu, po, nperseg, window, fs):
+    """Frames a quarter of a period apart: a bin of a pair is |A| + |B| = 2 |A|, whose square is out of range (3.4e38) where
+    |A|^2 = 1.7e38 is not. The scaled sum over the frames is in range at all of these sampling rates but the smallest, where
+    the amplitude is taken down by the scale's root."""
+    frames, hop, k0 = 1024, nperseg // 4, 9
+    w = np.ones(nperseg) if window == "boxcar" else 0.5 - 0.5 * np.cos(2 * np.pi * np.arange(nperseg) / nperseg)
+    scale = 1.0 / (fs * np.sum(w * w))
+    top = 1.3e19 if scale < 1 else 1.3e19 / np.sqrt(scale * frames * 4)
+    t = np.arange((frames - 1) * hop + nperseg)
+    x = (top / (0.5 * np.sum(w)) * np.cos(2 * np.pi * k0 * t / nperseg + 0.3)).astype(np.float32)
+    got = _welch(gpu, x, nperseg, nperseg - hop, window, False, fs)[1]
+    want = po.periodograms64(x.astype(np.float64), fs, nperseg, nperseg - hop, window=window, detrend=False).mean(axis=0)
+    assert np.all(np.isfinite(got)) and np.all(want < 3.4e38)
+    assert po.rel_l2(got, want) <= bound(nperseg)
