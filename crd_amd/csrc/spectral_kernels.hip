@@ -178,7 +178,8 @@ __global__ __launch_bounds__((SpecCfg<H, E>::threads)) void k_spec(SpecArgs a)
             const cf e = {(zk.x + zh.x) * 0.5f, (zk.y - zh.y) * 0.5f};
             const cf o = {(zk.y + zh.y) * 0.5f, (zh.x - zk.x) * 0.5f};
             // X[0] without its products: they are exact, but infinity times the zero parts would be NaN
-            const cf xk = m == 0 && k == 0 ? cf{zk.x + zk.y, 0.0f} : cadd(e, cmul(o, wk[k]));
+            const cf xk =
+                MODE == 0 && m == 0 && k == 0 ? cf{zk.x + zk.y, 0.0f} : cadd(e, cmul(o, wk[k]));
             // k == 0 also yields the Nyquist bin: W_N^H = -1, X[H] = Re Z0 - Im Z0 (read only where k == 0)
             const cf xn = {zk.x - zk.y, 0.0f};
             if constexpr (MODE == 0)
@@ -342,11 +343,14 @@ __global__ __launch_bounds__((WelchCfg<N, E>::threads)) void k_welch(SpecArgs a)
                 v[m] = csub(v[m], mean);
             }
         }
-#pragma unroll
-        for (int m = 0; m < E; ++m)
+        if (a.window != nullptr || a.scale != 1.0f)
         {
-            v[m].x *= win[m];
-            v[m].y *= win[m];
+#pragma unroll
+            for (int m = 0; m < E; ++m)
+            {
+                v[m].x *= win[m];
+                v[m].y *= win[m];
+            }
         }
         fft_core<N, E, false, 1>(v, i, view, reinterpret_cast<const cf*>(a.tw));
         // an idle lane group or half of a pair: the samples are zeros, less a mean of zero
