@@ -109,8 +109,10 @@ crdfft_status run(crdfft_spectral_plan p, const float* x, uint64_t len, int mode
     const float inv = static_cast<float>(1.0 / static_cast<double>(frames));
     // pairs of frames leave half as many lane groups to fill the chip: measured us of pairs / single frames at 50 % overlap,
     // nperseg 64: 256 frames 7.8 / 6.7, 512 6.8 / 8.0, 32768 8.9 / 172; 1024: 512 11.5 / 10.0, 1024 11.5 / 13.5, 32768
-    // 37 / 78; 4096: 512 15.3 / 13.1, 1024 16.8 / 20.9, 32768 168 / 225; 8192: 512 18.9 / 19.1, 1024 25.1 / 27.9
-    if (p->pair_wgs > 0 && frames >= (p->nperseg <= 256 ? 512u : 1024u))
+    // 37 / 78; 4096: 512 15.3 / 13.1, 1024 16.8 / 20.9, 32768 168 / 225. 8192: 768 24.4 / 23.9; one frame more than a round of
+    // lane groups (768 on 256 CUs) takes single frames a second round, 777 25.2 / 33.1, 1000 25.4 / 32.3
+    const uint64_t pairs_from = p->nperseg <= 256 ? 512 : p->nperseg <= 4096 ? 1024 : std::min<uint64_t>(p->welch_wgs + 1, 1024);
+    if (p->pair_wgs > 0 && frames >= pairs_from)
     {
         const uint64_t pairs = (frames + 1) / 2;
         const uint64_t wgs = std::min<uint64_t>((pairs + p->ppg - 1) / p->ppg, p->pair_wgs);

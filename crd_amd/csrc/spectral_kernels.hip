@@ -383,7 +383,7 @@ __global__ __launch_bounds__((WelchCfg<N, E>::threads)) void k_welch(SpecArgs a)
 }
 
 // acc[k] = ((first ? 0 : acc[k]) + sum over the rows of rows[r][k]) * scale, in a fixed order: a workgroup owns 64
-// bins, its 16 row groups sum rows g, g + 16, ... (four loads in flight per step), and the 16 partial sums are added
+// bins, its 16 row groups sum rows g, g + 16, ... (AHEAD loads in flight per step), and the 16 partial sums are added
 // in group order, so the result does not depend on timing. The sums carry their rounding errors along, so thousands of
 // rows add none of their own.
 constexpr int kSumBins = 64;
@@ -398,29 +398,36 @@ __device__ __forceinline__ void add_compensated(float& s, float& c, float x)
     s = t;
 }
 
-__global__ __launch_bounds__(kSumBins * kSumGroups) void k_spec_sum(const float* rows, float* acc, uint64_t nfreq,
-                                                                    uint64_t nrows, int first, float scale, float scale_lo)
+template <int AHEAD>
+__global__ __launch_bounds__(kSumBins * kSumGroups) void k_spec_sum(const float* rows, float* acc, uint32_t nfreq,
+                                                                    uint32_t nrows, int first, float scale, float scale_lo)
 {
     __shared__ float part[kSumGroups][kSumBins], rest[kSumGroups][kSumBins];
     const int kk = threadIdx.x % kSumBins;
     const int g = threadIdx.x / kSumBins;
-    const uint64_t k = static_cast<uint64_t>(blockIdx.x) * kSumBins + kk;
+    const uint32_t k = blockIdx.x * kSumBins + kk;
     float s = 0.0f, c = 0.0f;
     if (k < nfreq)
     {
-        uint64_t r = g;
-        for (; r + 3 * kSumGroups < nrows; r += 4 * kSumGroups)
+        // one 32-bit offset a load and no checks: a row past the last one reads zero
+        const __amdgpu_buffer_rsrc_t in = make_rsrc(rows, nrows * nfreq * 4u);
+        const uint32_t step = kSumGroups * nfreq * 4u;
+        uint32_t off = (g * nfreq + k) * 4u;
+        for (uint32_t r = 0; r < nrows; r += AHEAD * kSumGroups)
         {
-            const float x0 = rows[r * nfreq + k], x1 = rows[(r + kSumGroups) * nfreq + k];
-            const float x2 = rows[(r + 2 * kSumGroups) * nfreq + k], x3 = rows[(r + 3 * kSumGroups) * nfreq + k];
-            add_compensated(s, c, x0);
-            add_compensated(s, c, x1);
-            add_compensated(s, c, x2);
-            add_compensated(s, c, x3);
-        }
-        for (; r < nrows; r += kSumGroups)
-        {
-            add_compensated(s, c, rows[r * nfreq + k]);
+            float x[AHEAD];
+#pragma unroll
+            for (int q = 0; q < AHEAD; ++q)
+            {
+                x[q] = bld32<0>(in, off + q * step, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0); // all on their way before the first one is waited for
+#pragma unroll
+            for (int q = 0; q < AHEAD; ++q)
+            {
+                add_compensated(s, c, x[q]);
+            }
+            off += AHEAD * step;
         }
     }
     part[g][kk] = s;
@@ -573,8 +580,18 @@ hipError_t welch_pair_residency(uint64_t n, int* per_cu)
 hipError_t launch_spec_sum(const float* rows, float* acc, uint64_t nfreq, uint64_t nrows, bool first, float scale,
                            hipStream_t s, float scale_lo)
 {
-    hipLaunchKernelGGL(k_spec_sum, dim3(static_cast<unsigned>((nfreq + kSumBins - 1) / kSumBins)),
-                       dim3(kSumBins * kSumGroups), 0, s, rows, acc, nfreq, nrows, first ? 1 : 0, scale, scale_lo);
+    // the last step's offsets as well are 32 bits wide
+    if ((nrows + 2 * 8 * kSumGroups) * nfreq >= (uint64_t{1} << 30))
+    {
+        return hipErrorInvalidValue;
+    }
+    // Eight rows ahead where the few workgroups wait for memory (Welch us of 8 / 4 rows ahead: nperseg 4, 4096 frames
+    // 18.2 / 27.0, 1024, 1000 frames 11.5 / 14.2); four where one step of them covers the rows or the bins fill the chip
+    // (16, 1024 frames 10.1 / 9.9; 32768, 4096 frames 505 / 497).
+    const unsigned blocks = static_cast<unsigned>((nfreq + kSumBins - 1) / kSumBins);
+    auto kern = nrows > 4 * kSumGroups && blocks < 256 ? k_spec_sum<8> : k_spec_sum<4>;
+    hipLaunchKernelGGL(kern, dim3(blocks), dim3(kSumBins * kSumGroups), 0, s, rows, acc, static_cast<uint32_t>(nfreq),
+                       static_cast<uint32_t>(nrows), first ? 1 : 0, scale, scale_lo);
     return hipGetLastError();
 }
 

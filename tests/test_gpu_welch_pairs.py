@@ -1,5 +1,5 @@
 """Welch over pairs of frames (two frames per complex transform) at the frame counts where it takes over from single frames
-(512 up to 256 samples a frame, 1024 above), odd counts (half a pair), odd hops (frames on any 4-byte boundary) and both
+(512 up to 256 samples a frame, 1024 above, 769 at 8192 on 256 CUs), odd counts (half a pair), odd hops (frames on any 4-byte boundary) and both
 window / detrend settings, against the oracle's FP64 restatement: rel-L2 <= 2e-6 log2(nperseg), the bar of the spectral
 tests, also where a pair's squares would leave the range unscaled. A NaN sample reaches every bin, a zero signal gives zeros, reruns are bit-identical."""
 import numpy as np
@@ -34,7 +34,7 @@ def _welch(gpu, x, nperseg, noverlap, window, detrend, fs=250.0):
     (64, 63, 512, "hann", True), (128, 128, 40001, "hann", True), (256, 31, 513, "hann", True),
     (512, 7, 1023, "hann", True), (512, 7, 1024, "boxcar", True), (1024, 101, 1025, "hann", True),
     (2048, 2048, 1026, "hann", True), (4096, 64, 1024, "hann", True), (4096, 65, 5001, "hann", False),
-    (8192, 33, 1027, "hann", True)])
+    (8192, 33, 768, "hann", True), (8192, 33, 769, "hann", True), (8192, 33, 1027, "hann", True)])
 def test_pairs_match_fp64(gpu, po, nperseg, hop, frames, window, detrend):
     print(f"welch nperseg={nperseg} hop={hop} frames={frames} {window} {detrend}", flush=True)
     length = frames * hop + nperseg - hop + min(hop - 1, 2)  # samples past the last frame are not read
