@@ -834,13 +834,13 @@ crdfft_status execute_impl(crdfft_plan p, const void* in, void* out, int32_t dir
             if (sh.algorithm == CRDFFT_ALGO_SINGLE && (p->flags & CRDFFT_FLAG_SEPARATE_PASSES) == 0 && !p->floor &&
                 crdfft::spec_shape(h, &se, &per_group) && se == sh.e)
             {
-                // n <= 32768: load, half-length core, recombine and store in one launch (the spectral kernel's plain
-                // mode: no window, no detrend, frames = rows at idist); measured 1.2-2.1x the separate passes (2^25
+                // n <= 32768: load, half-length core, recombine and store in one launch (the spectral kernel's mode of plain
+                // rows, frames = rows at idist); measured 1.2-2.1x the separate passes (2^25
                 // points: n = 4 124 / 148 us, 16 105 / 115, 64 51 / 99, 256 46 / 93)
                 const crdfft::SpecArgs a{static_cast<const float*>(in), nullptr, p->wreal.as<cfloat>(),
                                          p->tw_single.as<cfloat>(), out, sh.batch, p->idist, 1.0f, 0, p->odist};
                 CRDFFT_TRY(prof.before());
-                CRDFFT_TRY(crdfft::launch_spec(h, 0, a, (sh.batch + per_group - 1) / per_group, s));
+                CRDFFT_TRY(crdfft::launch_spec(h, 3, a, (sh.batch + per_group - 1) / per_group, s));
                 CRDFFT_TRY(prof.after(0, h * sh.batch));
                 return CRDFFT_OK;
             }

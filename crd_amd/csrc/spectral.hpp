@@ -28,7 +28,8 @@ constexpr int kSpecWelchMaxH = 8192;
 
 // Values per thread and frames per workgroup of the kernel for H = nperseg / 2 (false: no instantiation).
 bool spec_shape(uint64_t h, int* e, unsigned* frames_per_group);
-// mode 0: complex rows (STFT); 1: density rows; 2: Welch partial rows, one per lane group. groups = workgroups.
+// mode 0: complex rows (STFT); 1: density rows; 2: Welch partial rows, one per lane group; 3: complex rows without window
+// and mean (R2C), SpecArgs::window nullptr and detrend 0. groups = workgroups.
 hipError_t launch_spec(uint64_t h, int mode, const SpecArgs& a, uint64_t groups, hipStream_t s);
 // Resident workgroups per CU of the Welch lane-group kernel (the persistent grid is this times the CU count).
 hipError_t spec_welch_residency(uint64_t h, int* per_cu);

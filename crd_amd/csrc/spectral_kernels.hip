@@ -13,6 +13,8 @@
 //   MODE 2  nothing per frame: lane group g sums the periodograms of frames g, g + G, g + 2G, ... in registers and
 //           writes one partial row; k_spec_sum adds the G partial rows in order (Welch, bit-identical run to run).
 //           Frames of 32768 samples run MODE 1 in chunks of rows instead, each chunk added in order.
+//   MODE 3  R2C rows below 512 points: X[0] as the plain sum, as the separate pass forms it. The product with W^0 = 1 is
+//           exact for finite values but makes NaN of an infinity; in the other modes and lengths the select costs 2-4 %.
 // HBM traffic: the signal once per frame that covers it (twice at 50% overlap) and the output; no framed copy of
 // the signal, no spectrum round trip.
 #include "buffer.hpp"
@@ -63,7 +65,7 @@ __global__ __launch_bounds__((SpecCfg<H, E>::threads)) void k_spec(SpecArgs a)
     {
         acc[m] = 0.0f;
     }
-    // MODE 0/1: one frame per lane group; MODE 2: frames group, group + groups, ... (uniform trip count per
+    // MODE 0/1/3: one frame per lane group; MODE 2: frames group, group + groups, ... (uniform trip count per
     // workgroup: every lane group runs the same number of iterations, idle ones on a masked frame)
     const uint64_t iters = MODE == 2 ? (a.frames + groups - 1) / groups : 1;
     // 8-byte sample pairs when every frame starts 8-byte aligned (an even hop from an 8-byte aligned signal)
@@ -103,7 +105,7 @@ __global__ __launch_bounds__((SpecCfg<H, E>::threads)) void k_spec(SpecArgs a)
                 v[m] = cf{xr.ld32(j, 8u * T * m), xr.ld32(j + 4u, 8u * T * m)};
             }
         }
-        if (a.detrend != 0)
+        if (MODE != 3 && a.detrend != 0)
         {
             // the frame mean, in a fixed order: a butterfly over the frame's lanes of one wave (each step adds the
             // same two partial sums in both lanes, so every lane ends with the same bits), then the waves' sums in
@@ -144,7 +146,7 @@ __global__ __launch_bounds__((SpecCfg<H, E>::threads)) void k_spec(SpecArgs a)
                 v[m].y -= mean;
             }
         }
-        if (a.window != nullptr)
+        if (MODE != 3 && a.window != nullptr)
         {
             const __amdgpu_buffer_rsrc_t wr = make_rsrc(win, 8u * H);
 #pragma unroll
@@ -177,12 +179,10 @@ __global__ __launch_bounds__((SpecCfg<H, E>::threads)) void k_spec(SpecArgs a)
                                  : (T >= 16 ? view.get_at(pad16(T - i), T * (E - 1 - m)) : view.get(H - k));
             const cf e = {(zk.x + zh.x) * 0.5f, (zk.y - zh.y) * 0.5f};
             const cf o = {(zk.y + zh.y) * 0.5f, (zh.x - zk.x) * 0.5f};
-            // X[0] without its products: they are exact, but infinity times the zero parts would be NaN
-            const cf xk =
-                MODE == 0 && m == 0 && k == 0 ? cf{zk.x + zk.y, 0.0f} : cadd(e, cmul(o, wk[k]));
+            const cf xk = MODE == 3 && m == 0 && k == 0 ? cf{zk.x + zk.y, 0.0f} : cadd(e, cmul(o, wk[k]));
             // k == 0 also yields the Nyquist bin: W_N^H = -1, X[H] = Re Z0 - Im Z0 (read only where k == 0)
             const cf xn = {zk.x - zk.y, 0.0f};
-            if constexpr (MODE == 0)
+            if constexpr (MODE == 0 || MODE == 3)
             {
                 if (active)
                 {
@@ -494,7 +494,8 @@ hipError_t launch_spec(uint64_t h, int mode, const SpecArgs& a, uint64_t groups,
         using C = SpecCfg<H, E>;                                                                                       \
         if (mode == 2 && H > kSpecWelchMaxH)                                                                           \
             return hipErrorInvalidValue;                                                                               \
-        auto kern = mode == 0 ? k_spec<H, E, 0>                                                                        \
+        auto kern = mode == 3 && H < 256 ? k_spec<H, E, (H < 256 ? 3 : 0)>                                             \
+                    : mode == 0 || mode == 3 ? k_spec<H, E, 0>                                                         \
                               : (mode == 1 ? k_spec<H, E, 1> : k_spec<H, E, (H <= kSpecWelchMaxH ? 2 : 1)>);        \
         hipError_t err = set_lds(kern, C::lds_bytes);                                                                  \
         if (err != hipSuccess)                                                                                         \

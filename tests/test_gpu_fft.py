@@ -234,11 +234,11 @@ def test_r2c_c2r_padded_rows(gpu, po, n, batch, pad_in, pad_out):
         assert po.rel_l2(yb[:, :n], po.irfft64(Y[:, : h + 1].astype(np.complex128), n)) <= bound(n)
 
 
-@pytest.mark.parametrize("n,batch", [(4, 3), (8, 70), (64, 5), (256, 9), (512, 3), (4096, 3), (32768, 3), (1 << 16, 256)])
+@pytest.mark.parametrize("n,batch", [(4, 3), (8, 70), (32, 9), (64, 5), (256, 9), (1 << 16, 256)])
 def test_r2c_of_non_finite_rows(gpu, n, batch):
-    """X[0] and X[n/2] are sums without products: real for every input (real_fft.hpp:40), and infinite where the only
-    non-finite sample is the infinity x[0] (up to one kernel's lengths; above, the twiddles come before the sums). Other
-    rows are untouched by a row of NaN."""
+    """X[0] and X[n/2] as sums without products (below 512 points and in the whole transforms of 2^16): real for every input
+    (real_fft.hpp:40), and infinite where the only non-finite sample is the infinity x[0] (below 512 points; above, the
+    twiddles come before the sums). Other rows are untouched by a row of NaN."""
     h = n // 2
     x = np.random.default_rng(n).standard_normal((batch, n)).astype(np.float32)
     x[0, 0] = np.inf
@@ -250,7 +250,7 @@ def test_r2c_of_non_finite_rows(gpu, n, batch):
     X = dst.download((batch, h + 1), np.complex64)
     assert not X[0, 0].imag and not X[0, h].imag and not X[1, 0].imag and not X[1, h].imag
     assert np.isnan(X[1, 0].real) and np.isnan(X[1, h].real)
-    if n <= 32768:
+    if n < 512:
         assert X[0, 0].real == np.inf and X[0, h].real == np.inf
     else:
         assert not np.isfinite(X[0, 0].real)
