@@ -178,7 +178,37 @@ template <int N, int E> struct RowCfg
     static constexpr int lds_bytes = RS * M * 4;
 };
 
-template <int N, int E, bool INV>
+// LATE: a stage's twiddles after its exchange and one LDS address per element, in place of fft_core's twiddles ahead and
+// shared addresses; the same results. Ahead is the faster form by 2-10 % (16384 points by 10 %), but a batch that the chip
+// holds at once reads in one burst and writes in another, and what gets its workgroups through the stages in step lets the
+// bursts meet less. Late over ahead, us at `points` per CU (256 CUs):
+//   E = 8    n = 1024: 8192 7.8 / 7.7, 12288 9.6 / 12.2, 14336 11.1 / 13.6, 16384 14.7 / 15.1, 18432 18.1 / 17.1, 32768 27.7 / 27.1;
+//            n = 2048: 12288 9.9 / 12.6, 16384 14.3 / 15.5, 18432 17.9 / 17.1; n = 256 and 512 (tuned) alike
+//   E = 16   n = 256: 8192 6.8 / 6.8, 12288 8.8 / 11.0, 16384 11.1 / 13.0, 18432 15.0 / 16.0, 24576 20.0 / 19.7, 32768 24.0 / 25.2,
+//            65536 45.7 / 45.8; n = 512: 12288 10.2 / 9.5, 16384 13.1 / 14.4, 18432 18.3 / 17.5, 32768 26.4 / 28.0, 65536 55.5 / 50.5;
+//            n = 1024..4096 (tuned) 14336: 8-11 % faster late, 12288 and 18432 0-10 % slower
+//   n = 4096, E = 8: 12288 10.5 / 11.8, 16384 12.7 / 16.3, 18432 19.0 / 18.5, 28672 26.1 / 25.9, 65536 55.6 / 54.8: always late
+//   E = 4 and 32, n = 128, 8192 and 16384: never slower ahead (8192 at E = 16 up to 1.4 % at 10240).
+template <int N, int E> constexpr bool kRowsHaveLate = (E == 8 && N >= 256 && N <= 4096) || (E == 16 && N >= 256 && N <= 4096);
+template <int N, int E> constexpr bool kRowsAlwaysLate = N == 4096 && E == 8;
+
+template <int N, int E> bool rows_late(uint64_t points, uint64_t cus)
+{
+    if (kRowsAlwaysLate<N, E> || !kRowsHaveLate<N, E>)
+    {
+        return kRowsAlwaysLate<N, E>;
+    }
+    const auto per_cu = [&](uint64_t above, uint64_t to) { return points > above * cus && points <= to * cus; };
+    if (E == 8)
+    {
+        return per_cu(8192, 16384);
+    }
+    return N == 256   ? per_cu(8192, 18432) || per_cu(24576, 32768)
+           : N == 512 ? per_cu(12288, 16384) || per_cu(24576, 32768)
+                      : per_cu(12288, 16384);
+}
+
+template <int N, int E, bool INV, bool LATE>
 __global__ __launch_bounds__((RowCfg<N, E>::threads)) void k_rows(RowArgs a)
 {
     using C = RowCfg<N, E>;
@@ -204,12 +234,7 @@ __global__ __launch_bounds__((RowCfg<N, E>::threads)) void k_rows(RowArgs a)
         }
     }
     const LdsView<1> view{lds + local * C::RS, C::LF};
-    // Twiddles ahead of the exchanges and shared LDS addresses, except for the four 512-thread workgroups a CU holds at n =
-    // 4096: a batch that fills the chip once reads in one burst and writes in another, and what gets its workgroups through
-    // the stages in step makes the bursts meet less (n = 4096 x 1024: 13.7 us without either, 14.1 with the shared addresses,
-    // 16.7 with both; x 256 6.8 / 6.6 / 6.1, x 4096 56.5 / 56.4 / 55.5).
-    constexpr bool kBurst = C::T == 512;
-    fft_core<N, E, INV, 1, E <= 16 && C::T >= 16 && !kBurst, !kBurst>(v, i, view, reinterpret_cast<const cf*>(a.tw));
+    fft_core<N, E, INV, 1, E <= 16 && C::T >= 16 && !LATE, !LATE>(v, i, view, reinterpret_cast<const cf*>(a.tw));
     if (active)
     {
         store_strided<E>(v, reinterpret_cast<cf*>(a.out) + t * a.odist + i, static_cast<uint32_t>(C::T), a.scale,
@@ -1173,7 +1198,9 @@ hipError_t launch_rows(uint64_t n, int e, bool inverse, const RowArgs& a, hipStr
     if (n == N && e == E)                                                                                              \
     {                                                                                                                  \
         using C = RowCfg<N, E>;                                                                                        \
-        auto kern = inverse ? k_rows<N, E, true> : k_rows<N, E, false>;                                                \
+        constexpr bool kLate = kRowsHaveLate<N, E>, kAhead = !kRowsAlwaysLate<N, E>;                                   \
+        auto kern = rows_late<N, E>(a.count * N, a.cus) ? (inverse ? k_rows<N, E, true, kLate> : k_rows<N, E, false, kLate>)  \
+                                                        : (inverse ? k_rows<N, E, true, !kAhead> : k_rows<N, E, false, !kAhead>); \
         hipError_t err = set_lds(kern, C::lds_bytes);                                                                  \
         if (err != hipSuccess)                                                                                         \
             return err;                                                                                                \

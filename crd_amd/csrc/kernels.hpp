@@ -26,6 +26,7 @@ struct RowArgs
     uint64_t odist;
     float scale; // applied to every output (1 = unscaled, exact)
     uint32_t hints; // kHintNtLoad / kHintNtStore
+    uint32_t cus = 256; // of the device (the launcher's choice of form)
 };
 
 // Cache hints: non-temporal loads of the input / stores of the output (streamed data that should not displace a

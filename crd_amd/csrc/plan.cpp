@@ -142,6 +142,7 @@ struct crdfft_plan_s
     // four-step twiddle of 256 x complex_n / 256; whole_cus > 0 when the plan has it
     DeviceBuffer whole_roots, whole_full;
     uint32_t whole_cus = 0;
+    uint32_t cus = 256; // of the device
     bool whole_always = false; // the self-check's plan of one transform: whatever the batch
     uint32_t hshift = 0;
     DeviceBuffer wreal;     // W_n^k, k <= n/2, for R2C/C2R
@@ -465,7 +466,7 @@ crdfft_status run_complex(crdfft_plan_s* p, const cfloat* in, cfloat* out, uint6
             return CRDFFT_OK;
         case CRDFFT_ALGO_SINGLE:
         {
-            crdfft::RowArgs a{in, out, p->tw_single.as<cfloat>(), count, idist, odist, scale, sh.hints};
+            crdfft::RowArgs a{in, out, p->tw_single.as<cfloat>(), count, idist, odist, scale, sh.hints, p->cus};
             CRDFFT_TRY(prof.before());
             CRDFFT_TRY(crdfft::launch_rows(cn, sh.e, inverse, a, s));
             CRDFFT_TRY(prof.after(0, cn * count));
@@ -965,13 +966,11 @@ crdfft_status create_plan(crdfft_plan* plan, uint64_t n, uint64_t batch, uint64_
     p->odist = odist;
     p->flags = flags;
     (void)hipGetDevice(&p->device);
-    if (shape.whole && (type == CRDFFT_C2C || (flags & CRDFFT_FLAG_SEPARATE_PASSES) == 0))
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, p->device) == hipSuccess && cus > 0)
     {
-        int cus = 0;
-        if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, p->device) == hipSuccess && cus > 0)
-        {
-            p->whole_cus = static_cast<uint32_t>(cus);
-        }
+        p->cus = static_cast<uint32_t>(cus);
+        p->whole_cus = shape.whole && (type == CRDFFT_C2C || (flags & CRDFFT_FLAG_SEPARATE_PASSES) == 0) ? p->cus : 0u;
     }
     crdfft_status rs = build_tables(p, nullptr);
     if (rs == CRDFFT_OK)

@@ -56,6 +56,33 @@ def test_odd_batches_and_in_place(gpu, po, n, batch):
     assert po.rel_l2(y, po.fft64_of_f32(x)) <= bound(n)
 
 
+# the launch picks the twiddles' place by the points per CU (256): above 8192 to 16384 late at 8 values per thread; at 16
+# values 256 points above 8192 to 18432 and above 24576 to 32768, 512 points above 12288 to 16384 and above 24576 to 32768
+@pytest.mark.parametrize("n,ahead,late", [(256, 8192, (8193, 18432, 24577, 32768)), (512, 6144, (6145, 8192, 12289, 16384)),
+                                          (1024, 2048, (2049, 4096)), (2048, 1024, (1025, 2048))])
+@pytest.mark.parametrize("inverse", [False, True])
+def test_late_and_early_twiddles_are_bit_identical(gpu, po, n, ahead, late, inverse):
+    print(f"rows n={n} ahead={ahead} late={late} inverse={inverse}", flush=True)
+    direction = gpu.INVERSE if inverse else gpu.FORWARD
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal((late[-1] + 1, 2 * n), dtype=np.float32).view(np.complex64)
+    src, dst = gpu.DeviceBuffer.from_array(x), gpu.DeviceBuffer(x.nbytes)
+    early, want = gpu.FftPlan(n, ahead), np.empty_like(x)
+    part = gpu.DeviceBuffer(8 * n * ahead)
+    for first in range(0, len(x), ahead):
+        first = min(first, len(x) - ahead)
+        early.execute(src.address + 8 * n * first, part, direction)
+        gpu.synchronize()
+        want[first:first + ahead] = part.download((ahead, n), np.complex64)
+    assert po.rel_l2(want[:64], po.fft64_of_f32(x[:64], inverse=inverse)) <= bound(n)
+    for batch in late + (late[-1] + 1,):
+        dst.fill(0)
+        gpu.FftPlan(n, batch).execute(src, dst, direction)
+        gpu.synchronize()
+        got = dst.download((batch, n), np.complex64)
+        assert np.array_equal(got.view(np.uint32), want[:batch].view(np.uint32)), batch
+
+
 def test_rerun_is_bit_identical(gpu, po):
     for n in (4096, 1 << 16):
         x = po.lcg_complex(n * 6, 3).reshape(6, n)
