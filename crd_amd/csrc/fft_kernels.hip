@@ -182,28 +182,34 @@ template <int N, int E> struct RowCfg
 // shared addresses; the same results. Ahead is the faster form by 2-10 % (16384 points by 10 %), but a batch that the chip
 // holds at once reads in one burst and writes in another, and what gets its workgroups through the stages in step lets the
 // bursts meet less. Late over ahead, us at `points` per CU (256 CUs):
-//   E = 8    n = 1024: 8192 7.8 / 7.7, 12288 9.6 / 12.2, 14336 11.1 / 13.6, 16384 14.7 / 15.1, 18432 18.1 / 17.1, 32768 27.7 / 27.1;
-//            n = 2048: 12288 9.9 / 12.6, 16384 14.3 / 15.5, 18432 17.9 / 17.1; n = 256 and 512 (tuned) alike
-//   E = 16   n = 256: 8192 6.8 / 6.8, 12288 8.8 / 11.0, 16384 11.1 / 13.0, 18432 15.0 / 16.0, 24576 20.0 / 19.7, 32768 24.0 / 25.2,
-//            65536 45.7 / 45.8; n = 512: 12288 10.2 / 9.5, 16384 13.1 / 14.4, 18432 18.3 / 17.5, 32768 26.4 / 28.0, 65536 55.5 / 50.5;
+//   E = 8    n = 1024: 8192 7.8 / 7.7, 12288 9.6 / 12.2, 14336 11.1 / 13.6, 16384 14.7 / 15.1, 18432 18.1 / 17.1, 32768 27.7 /
+//            27.1; n = 2048: 12288 9.9 / 12.6, 16384 14.3 / 15.5, 18432 17.9 / 17.1; n = 256 and 512 (tuned) alike
+//   E = 16   n = 256: 8192 6.8 / 6.8, 12288 8.8 / 11.0, 16384 11.1 / 13.0, 18432 15.0 / 16.0, 20480 17.6 / 17.8, 24576 20.0 /
+//            19.7, 32768 24.0 / 25.2, 65536 45.7 / 45.8; n = 512: 12288 10.2 / 9.5, 16384 13.1 / 14.4, 18432 18.3 / 17.5, 32768 26.4 / 28.0, 65536 55.5 / 50.5;
 //            n = 1024..4096 (tuned) 14336: 8-11 % faster late, 12288 and 18432 0-10 % slower
 //   n = 4096, E = 8: 12288 10.5 / 11.8, 16384 12.7 / 16.3, 18432 19.0 / 18.5, 28672 26.1 / 25.9, 65536 55.6 / 54.8: always late
 //   E = 4 and 32, n = 128, 8192 and 16384: never slower ahead (8192 at E = 16 up to 1.4 % at 10240).
 template <int N, int E> constexpr bool kRowsHaveLate = (E == 8 && N >= 256 && N <= 4096) || (E == 16 && N >= 256 && N <= 4096);
 template <int N, int E> constexpr bool kRowsAlwaysLate = N == 4096 && E == 8;
 
-template <int N, int E> bool rows_late(uint64_t points, uint64_t cus)
+// nd: rows that are one pass of an N-D transform, whose input the pass before or a copy has left in the caches: ahead from 512
+// points on (2048 x 2048 44.3 late, 42.5 ahead; 512 x 512 x 16 50.7 / 49.2), as above at 256 (256 x 256 x 72 45.5 / 45.9).
+template <int N, int E> bool rows_late(uint64_t points, uint64_t cus, bool nd)
 {
     if (kRowsAlwaysLate<N, E> || !kRowsHaveLate<N, E>)
     {
         return kRowsAlwaysLate<N, E>;
+    }
+    if (nd && N > 256)
+    {
+        return false;
     }
     const auto per_cu = [&](uint64_t above, uint64_t to) { return points > above * cus && points <= to * cus; };
     if (E == 8)
     {
         return per_cu(8192, 16384);
     }
-    return N == 256   ? per_cu(8192, 18432) || per_cu(24576, 32768)
+    return N == 256   ? per_cu(8192, 20480) || per_cu(24576, 32768)
            : N == 512 ? per_cu(12288, 16384) || per_cu(24576, 32768)
                       : per_cu(12288, 16384);
 }
@@ -257,7 +263,33 @@ template <int N1, int E, int CC> struct ColCfg
 // PRE (C2R, INV): the column values are formed from the h + 1 input bins as pre_scale * Z[j] (c2r_z) on load, which
 // replaces the separate pre-rotation pass; X[h-j] of a column lies in the mirrored column, read in the same
 // coalesced pattern backwards.
-template <int N1, int E, int CC, bool INV, bool PRE = false>
+// LATE: as in k_rows. Late / ahead, us of the whole call at points per CU:
+//   four-step, forward: n = 2^16 (n1 = 256) 12288 20.3 / 20.2, 12800 23.5 / 25.5, 14336 24.3 / 27.0, 16384 26.4 / 28.9, 16896
+//     30.9 / 31.4; 2^17 (256) 12288 22.8 / 22.5, 14336 25.4 / 28.5, 16384 27.5 / 30.0, 16896 34.5 / 35.0; 2^15 (128) 12288 20.1 /
+//     19.9, 12800 22.9 / 24.4, 15360 25.4 / 27.2 (whole transforms from 16384 on). Inverse: 2^15 alike, 2^16 and 2^17 within 2 %
+//     either way.
+//   without a twiddle, in place, several matrices (N-D, a copy of the volume included) with rows of 256 columns and more: 256 x
+//     256 14336 42.6 / 43.1, 16384 45.2 / 45.1, 18432 46.1 / 49.8, 22528 52.6 / 55.9, 24576 57.6 / 58.4, 32768 71.4 / 71.8;
+//     128 x 256 16384 46.2 / 45.8, 17408 42.4 / 47.7, 18432 44.7 / 47.4, 20480 48.1 / 48.5, 22528 53.4 / 53.2. Rows of 64 and 128
+//     columns and single matrices: never slower ahead.
+// From n1 = 512 on never slower ahead.
+template <int N1, int E, int CC> constexpr bool kColsHaveLate = (N1 == 128 || N1 == 256) && E == 16 && CC == 16;
+
+template <int N1, int E, int CC> bool cols_late(const ColArgs& a, bool inverse)
+{
+    const uint64_t points = a.count * a.ncols * N1, cus = a.cus;
+    if (!kColsHaveLate<N1, E, CC>)
+    {
+        return false;
+    }
+    if (a.tfull != nullptr)
+    {
+        return (!inverse || N1 == 128) && points > 12288 * cus && points <= 16384 * cus;
+    }
+    return a.thi == nullptr && a.count > 1 && a.ncols >= 256 && points > 16384 * cus && points <= (N1 == 128 ? 20480 : 24576) * cus;
+}
+
+template <int N1, int E, int CC, bool INV, bool PRE = false, bool LATE = false>
 __global__ __launch_bounds__((ColCfg<N1, E, CC>::threads)) void k_cols(ColArgs a)
 {
     using C = ColCfg<N1, E, CC>;
@@ -306,7 +338,7 @@ __global__ __launch_bounds__((ColCfg<N1, E, CC>::threads)) void k_cols(ColArgs a
         }
     }
     const LdsView<CC> view{lds + c, C::IM};
-    fft_core<N1, E, INV, CC>(v, i, view, reinterpret_cast<const cf*>(a.tw));
+    fft_core<N1, E, INV, CC, E <= 16 && C::T >= 16 && !LATE, !LATE>(v, i, view, reinterpret_cast<const cf*>(a.tw));
     if (!active)
     {
         return;
@@ -1199,7 +1231,7 @@ hipError_t launch_rows(uint64_t n, int e, bool inverse, const RowArgs& a, hipStr
     {                                                                                                                  \
         using C = RowCfg<N, E>;                                                                                        \
         constexpr bool kLate = kRowsHaveLate<N, E>, kAhead = !kRowsAlwaysLate<N, E>;                                   \
-        auto kern = rows_late<N, E>(a.count * N, a.cus) ? (inverse ? k_rows<N, E, true, kLate> : k_rows<N, E, false, kLate>)  \
+        auto kern = rows_late<N, E>(a.count * N, a.cus, a.nd) ? (inverse ? k_rows<N, E, true, kLate> : k_rows<N, E, false, kLate>)  \
                                                         : (inverse ? k_rows<N, E, true, !kAhead> : k_rows<N, E, false, !kAhead>); \
         hipError_t err = set_lds(kern, C::lds_bytes);                                                                  \
         if (err != hipSuccess)                                                                                         \
@@ -1231,7 +1263,10 @@ hipError_t launch_cols(uint64_t n1, int e, int c, bool inverse, const ColArgs& a
         using C = ColCfg<N, E, CC>;                                                                                    \
         if (static_cast<uint64_t>(N) * a.ncols >= (uint64_t{1} << 32))                                                 \
             return hipErrorInvalidValue; /* the kernel's in-matrix offsets are 32-bit */                               \
-        auto kern = inverse ? k_cols<N, E, CC, true> : k_cols<N, E, CC, false>;                                        \
+        constexpr bool kLate = kColsHaveLate<N, E, CC>;                                                                \
+        auto kern = cols_late<N, E, CC>(a, inverse)                                                                \
+                        ? (inverse ? k_cols<N, E, CC, true, false, kLate> : k_cols<N, E, CC, false, false, kLate>)     \
+                        : (inverse ? k_cols<N, E, CC, true> : k_cols<N, E, CC, false>);                                \
         hipError_t err = set_lds(kern, C::lds_bytes);                                                                  \
         if (err != hipSuccess)                                                                                         \
             return err;                                                                                                \

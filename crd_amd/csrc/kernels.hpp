@@ -26,7 +26,9 @@ struct RowArgs
     uint64_t odist;
     float scale; // applied to every output (1 = unscaled, exact)
     uint32_t hints; // kHintNtLoad / kHintNtStore
-    uint32_t cus = 256; // of the device (the launcher's choice of form)
+    // the launcher's choice of form: CUs of the device, and whether the rows are one pass of an N-D transform
+    uint32_t cus = 256;
+    bool nd = false;
 };
 
 // Cache hints: non-temporal loads of the input / stores of the output (streamed data that should not displace a
@@ -65,6 +67,7 @@ struct ColArgs
     // formed as pre_scale * Z[j] from X[j], X[h-j] and wreal[j] = W_n^j on load
     const cfloat* wreal = nullptr;
     float pre_scale = 1.0f;
+    uint32_t cus = 256; // of the device (the launcher's choice of form)
 };
 
 // Row transforms of length n2 over the n1 rows of a row-major n1 x n2 matrix, stored transposed:

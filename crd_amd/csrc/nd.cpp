@@ -92,7 +92,12 @@ crdfft_status line_plan(uint64_t d, uint64_t lines, crdfft_plan* out, bool* blue
     {
         return crdfft_bluestein_plan_create(out, d, lines, d, d, 0);
     }
-    return crdfft_plan_create(out, d, lines, d, d, CRDFFT_C2C, CRDFFT_FP32, CRDFFT_FLAG_NO_SELF_CHECK);
+    const crdfft_status st = crdfft_plan_create(out, d, lines, d, d, CRDFFT_C2C, CRDFFT_FP32, CRDFFT_FLAG_NO_SELF_CHECK);
+    if (st == CRDFFT_OK)
+    {
+        crdfft::plan_set_nd_pass(*out);
+    }
+    return st;
 }
 
 crdfft_status build(crdfft_nd_plan_s* p, const uint64_t* dims, uint32_t ndim, uint64_t batch, uint32_t flags)

@@ -143,6 +143,7 @@ struct crdfft_plan_s
     DeviceBuffer whole_roots, whole_full;
     uint32_t whole_cus = 0;
     uint32_t cus = 256; // of the device
+    bool nd_pass = false; // the rows of an N-D plan
     bool whole_always = false; // the self-check's plan of one transform: whatever the batch
     uint32_t hshift = 0;
     DeviceBuffer wreal;     // W_n^k, k <= n/2, for R2C/C2R
@@ -466,7 +467,7 @@ crdfft_status run_complex(crdfft_plan_s* p, const cfloat* in, cfloat* out, uint6
             return CRDFFT_OK;
         case CRDFFT_ALGO_SINGLE:
         {
-            crdfft::RowArgs a{in, out, p->tw_single.as<cfloat>(), count, idist, odist, scale, sh.hints, p->cus};
+            crdfft::RowArgs a{in, out, p->tw_single.as<cfloat>(), count, idist, odist, scale, sh.hints, p->cus, p->nd_pass};
             CRDFFT_TRY(prof.before());
             CRDFFT_TRY(crdfft::launch_rows(cn, sh.e, inverse, a, s));
             CRDFFT_TRY(prof.after(0, cn * count));
@@ -569,7 +570,8 @@ crdfft_status run_complex(crdfft_plan_s* p, const cfloat* in, cfloat* out, uint6
                                        cn,
                                        (sh.hints & crdfft::kHintNtLoad) | tiled,
                                        c2r_w,
-                                       1.0f / static_cast<float>(cn)};
+                                       1.0f / static_cast<float>(cn),
+                                       p->cus};
                     CRDFFT_TRY(prof.before());
                     if (c2r_w != nullptr)
                     {
@@ -1252,6 +1254,8 @@ crdfft_status plan_use_floor(crdfft_plan p)
     p->floor = true;
     return CRDFFT_OK;
 }
+
+void plan_set_nd_pass(crdfft_plan p) { p->nd_pass = true; }
 
 bool plan_uses_whole(crdfft_plan p) { return p->whole_cus > 0 && whole_of(p, p->shape.batch) > 0; }
 

@@ -95,6 +95,9 @@ constexpr uint32_t kCoopSpinLimit = 1u << 18;
 crdfft_status plan_use_floor(crdfft_plan p);
 bool plan_on_floor(crdfft_plan p);
 
+// The plan runs the rows of an N-D plan (RowArgs::nd).
+void plan_set_nd_pass(crdfft_plan p);
+
 // Plans with PlanShape::whole: whether any of their batch runs on the whole-transform kernel, and switching a self-check's
 // one-transform plan onto it.
 bool plan_uses_whole(crdfft_plan p);

@@ -57,8 +57,8 @@ def test_odd_batches_and_in_place(gpu, po, n, batch):
 
 
 # the launch picks the twiddles' place by the points per CU (256): above 8192 to 16384 late at 8 values per thread; at 16
-# values 256 points above 8192 to 18432 and above 24576 to 32768, 512 points above 12288 to 16384 and above 24576 to 32768
-@pytest.mark.parametrize("n,ahead,late", [(256, 8192, (8193, 18432, 24577, 32768)), (512, 6144, (6145, 8192, 12289, 16384)),
+# values 256 points above 8192 to 20480 and above 24576 to 32768, 512 points above 12288 to 16384 and above 24576 to 32768
+@pytest.mark.parametrize("n,ahead,late", [(256, 8192, (8193, 20480, 24577, 32768)), (512, 6144, (6145, 8192, 12289, 16384)),
                                           (1024, 2048, (2049, 4096)), (2048, 1024, (1025, 2048))])
 @pytest.mark.parametrize("inverse", [False, True])
 def test_late_and_early_twiddles_are_bit_identical(gpu, po, n, ahead, late, inverse):
@@ -81,6 +81,45 @@ def test_late_and_early_twiddles_are_bit_identical(gpu, po, n, ahead, late, inve
         gpu.synchronize()
         got = dst.download((batch, n), np.complex64)
         assert np.array_equal(got.view(np.uint32), want[:batch].view(np.uint32)), batch
+
+
+# the column kernels of 128 and 256 points likewise: four-step forward above 12288 to 16384 points per CU (tuned: 2^15 runs
+# whole transforms there), columns without a twiddle from rows of 256 columns above 16384 to 20480 / 24576
+@pytest.mark.parametrize("n,batches", [(1 << 15, (96, 97, 128, 129)), (1 << 16, (48, 49, 64, 65)), (1 << 17, (24, 25, 32, 33))])
+def test_late_and_early_columns_are_bit_identical(gpu, po, n, batches):
+    print(f"columns n={n} batches={batches}", flush=True)
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal((batches[-1], 2 * n), dtype=np.float32).view(np.complex64)
+    src, dst = gpu.DeviceBuffer.from_array(x), gpu.DeviceBuffer(x.nbytes)
+    for direction in (gpu.FORWARD, gpu.INVERSE):
+        want = None
+        for batch in batches:
+            gpu.FftPlan(n, batch, tuning={"chunk": 4096}).execute(src, dst, direction)
+            gpu.synchronize()
+            got = dst.download((batch, n), np.complex64)
+            want = got if want is None else want
+            rows = min(len(want), batch)
+            assert np.array_equal(got[:rows].view(np.uint32), want[:rows].view(np.uint32)), batch
+            ref = po.fft64_of_f32(x[batch - 1:batch], inverse=direction == gpu.INVERSE)
+            assert po.rel_l2(got[batch - 1:], ref) <= bound(n)
+
+
+@pytest.mark.parametrize("dims,batches", [((128, 256), (128, 129, 160, 161)), ((256, 256), (64, 65, 96, 97))])
+def test_late_and_early_nd_columns_are_bit_identical(gpu, dims, batches):
+    print(f"nd dims={dims} batches={batches}", flush=True)
+    rng = np.random.default_rng(dims[0])
+    x = rng.standard_normal((batches[-1], dims[0], 2 * dims[1]), dtype=np.float32).view(np.complex64)
+    want = None
+    for batch in batches:
+        buf = gpu.DeviceBuffer.from_array(x[:batch])
+        gpu.NdFftPlan(dims, batch).execute(buf, gpu.FORWARD)
+        gpu.synchronize()
+        got = buf.download((batch,) + dims, np.complex64)
+        want = got if want is None else want
+        rows = min(len(want), batch)
+        assert np.array_equal(got[:rows].view(np.uint32), want[:rows].view(np.uint32)), batch
+        ref = np.fft.fft2(x[batch - 1].astype(np.complex128))
+        assert np.linalg.norm(got[-1] - ref) <= bound(dims[0] * dims[1]) * np.linalg.norm(ref)
 
 
 def test_rerun_is_bit_identical(gpu, po):
