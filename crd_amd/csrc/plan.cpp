@@ -1259,11 +1259,11 @@ void plan_set_nd_pass(crdfft_plan p) { p->nd_pass = true; }
 
 bool plan_uses_whole(crdfft_plan p) { return p->whole_cus > 0 && whole_of(p, p->shape.batch) > 0; }
 
-crdfft_status plan_use_whole(crdfft_plan p)
+crdfft_status plan_set_whole(crdfft_plan p, bool on)
 {
-    p->whole_cus = 1;
-    p->whole_always = true;
-    return build_whole_tables(p, nullptr);
+    p->whole_cus = on ? 1 : 0;
+    p->whole_always = on;
+    return on && p->whole_full.ptr == nullptr ? build_whole_tables(p, nullptr) : CRDFFT_OK;
 }
 
 bool plan_on_floor(crdfft_plan p) { return p != nullptr && p->floor; }

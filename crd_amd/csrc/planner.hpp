@@ -99,8 +99,8 @@ bool plan_on_floor(crdfft_plan p);
 void plan_set_nd_pass(crdfft_plan p);
 
 // Plans with PlanShape::whole: whether any of their batch runs on the whole-transform kernel, and switching a self-check's
-// one-transform plan onto it.
+// one-transform plan onto it and back.
 bool plan_uses_whole(crdfft_plan p);
-crdfft_status plan_use_whole(crdfft_plan p);
+crdfft_status plan_set_whole(crdfft_plan p, bool on);
 
 } // namespace crdfft

@@ -130,6 +130,12 @@ extern "C" crdfft_status crdfft_self_check(crdfft_plan plan)
         // the plan's batch (three cases run as three calls of one transform each when the batch is 1)
         const uint64_t cases = 3;
         std::vector<std::complex<float>> host(n), out(n);
+        std::vector<std::complex<double>> root(n); // exp(2 pi i k / n)
+        for (uint64_t k = 0; k < n; ++k)
+        {
+            const double a = kTwoPi * static_cast<double>(k) / static_cast<double>(n);
+            root[k] = std::complex<double>(std::cos(a), std::sin(a));
+        }
         DevBuf din, dout;
         if (crdfft::device_malloc(&din.p, n * 8) != hipSuccess || crdfft::device_malloc(&dout.p, n * 8) != hipSuccess)
         {
@@ -144,19 +150,8 @@ extern "C" crdfft_status crdfft_self_check(crdfft_plan plan)
             return st;
         }
         crdfft_status result = CRDFFT_OK;
-        // both directions on the four-step or single kernel, then on the whole-transform kernel
-        for (int form = 0; form < (whole ? 4 : 2) && result == CRDFFT_OK; ++form)
+        for (int dir = 0; dir < 2 && result == CRDFFT_OK; ++dir)
         {
-            const int dir = form & 1;
-            const bool fault = fault_forced(plan, whole && form < 2);
-            if (form == 2)
-            {
-                result = crdfft::plan_use_whole(one);
-                if (result != CRDFFT_OK)
-                {
-                    break;
-                }
-            }
             for (uint64_t c = 0; c < cases && result == CRDFFT_OK; ++c)
             {
                 for (uint64_t j = 0; j < n; ++j)
@@ -167,9 +162,9 @@ extern "C" crdfft_status crdfft_self_check(crdfft_plan plan)
                     }
                     else if (c == 1)
                     {
-                        const double a = (dir == 0 ? 1.0 : -1.0) * kTwoPi * static_cast<double>((3 * j) % n) /
-                                         static_cast<double>(n);
-                        host[j] = std::complex<float>(static_cast<float>(std::cos(a)), static_cast<float>(std::sin(a)));
+                        const std::complex<double>& r = root[(3 * j) % n];
+                        host[j] = std::complex<float>(static_cast<float>(r.real()),
+                                                      static_cast<float>(dir == 0 ? r.imag() : -r.imag()));
                     }
                     else
                     {
@@ -181,57 +176,50 @@ extern "C" crdfft_status crdfft_self_check(crdfft_plan plan)
                     result = CRDFFT_HIP_ERROR;
                     break;
                 }
-                st = crdfft_execute(one, din.p, dout.p, dir, nullptr);
-                if (st != CRDFFT_OK)
+                // on the four-step or single kernel, then on the whole-transform kernel
+                for (int form = 0; form < (whole ? 2 : 1) && result == CRDFFT_OK; ++form)
                 {
-                    result = st;
-                    break;
-                }
-                if (hipMemcpy(out.data(), dout.p, n * 8, hipMemcpyDeviceToHost) != hipSuccess)
-                {
-                    result = CRDFFT_HIP_ERROR;
-                    break;
-                }
-                if (fault && c == 0)
-                {
-                    uint32_t bits;
-                    std::memcpy(&bits, &out[n - 1], 4);
-                    bits ^= 0x00400000u;
-                    std::memcpy(&out[n - 1], &bits, 4);
-                }
-                const double maxref = (c == 0) ? 1.0 : static_cast<double>(n);
-                double maxerr = 0.0;
-                for (uint64_t k = 0; k < n; ++k)
-                {
-                    if (!checked(k, n))
+                    if (whole)
                     {
-                        continue;
+                        st = crdfft::plan_set_whole(one, form == 1);
+                        if (st != CRDFFT_OK)
+                        {
+                            result = st;
+                            break;
+                        }
                     }
-                    std::complex<double> want(0.0, 0.0);
-                    if (c == 0)
+                    st = crdfft_execute(one, din.p, dout.p, dir, nullptr);
+                    if (st != CRDFFT_OK)
                     {
-                        const double a = -(dir == 0 ? 1.0 : -1.0) * kTwoPi * static_cast<double>(k % n) /
-                                         static_cast<double>(n);
-                        want = std::complex<double>(std::cos(a), std::sin(a));
+                        result = st;
+                        break;
                     }
-                    else if (c == 1)
+                    if (hipMemcpy(out.data(), dout.p, n * 8, hipMemcpyDeviceToHost) != hipSuccess)
                     {
-                        want = (k == 3 % n) ? std::complex<double>(static_cast<double>(n), 0.0) : want;
+                        result = CRDFFT_HIP_ERROR;
+                        break;
                     }
-                    else
+                    if (fault_forced(plan, whole && form == 0) && c == 0)
                     {
-                        want = (k == 0) ? std::complex<double>(static_cast<double>(n), 0.0) : want;
+                        uint32_t bits;
+                        std::memcpy(&bits, &out[n - 1], 4);
+                        bits ^= 0x00400000u;
+                        std::memcpy(&out[n - 1], &bits, 4);
                     }
-                    const std::complex<double> got(out[k].real(), out[k].imag());
-                    const double err = std::abs(got - want);
-                    if (!(err <= maxerr))
+                    const double maxref = (c == 0) ? 1.0 : static_cast<double>(n);
+                    const double limit = tol * (1.0 + maxref);
+                    const uint64_t peak = c == 1 ? 3 % n : 0;
+                    for (uint64_t k = 0; k < n && result == CRDFFT_OK; ++k)
                     {
-                        maxerr = err; // NaN also lands here and fails below
+                        double re = c == 0 ? root[k].real() : (k == peak ? maxref : 0.0);
+                        double im = c == 0 ? (dir == 0 ? -root[k].imag() : root[k].imag()) : 0.0;
+                        re -= out[k].real();
+                        im -= out[k].imag();
+                        if (!(re * re + im * im <= limit * limit) && checked(k, n)) // NaN as well
+                        {
+                            result = CRDFFT_SELF_CHECK_FAILED;
+                        }
                     }
-                }
-                if (!(maxerr <= tol * (1.0 + maxref)))
-                {
-                    result = CRDFFT_SELF_CHECK_FAILED;
                 }
             }
         }
@@ -253,13 +241,18 @@ extern "C" crdfft_status crdfft_self_check(crdfft_plan plan)
         return st;
     }
     crdfft_status result = CRDFFT_OK;
+    std::vector<double> cosine(n);
+    for (uint64_t j = 0; j < n; ++j)
+    {
+        cosine[j] = std::cos(kTwoPi * static_cast<double>(j) / static_cast<double>(n));
+    }
     // on the four-step or single kernel, then on the whole-transform kernel
     for (int form = 0; form < (whole ? 2 : 1) && result == CRDFFT_OK; ++form)
     {
         const bool fault = fault_forced(plan, whole && form == 0);
-        if (form == 1)
+        if (whole)
         {
-            result = crdfft::plan_use_whole(one);
+            result = crdfft::plan_set_whole(one, form == 1);
             if (result != CRDFFT_OK)
             {
                 break;
@@ -267,11 +260,7 @@ extern "C" crdfft_status crdfft_self_check(crdfft_plan plan)
         }
         if (info.type == CRDFFT_R2C)
         {
-            std::vector<float> x(n);
-            for (uint64_t j = 0; j < n; ++j)
-            {
-                x[j] = static_cast<float>(std::cos(kTwoPi * static_cast<double>(j) / static_cast<double>(n)));
-            }
+            std::vector<float> x(cosine.begin(), cosine.end());
             std::vector<std::complex<float>> X(h + 1);
             if (hipMemcpy(dr.p, x.data(), n * 4, hipMemcpyHostToDevice) != hipSuccess)
             {
@@ -291,23 +280,14 @@ extern "C" crdfft_status crdfft_self_check(crdfft_plan plan)
                 {
                     X[1] = std::complex<float>(X[1].real() * 1.5f, X[1].imag());
                 }
-                double maxerr = 0.0;
-                for (uint64_t k = 0; k <= h; ++k)
+                const double limit = tol * (1.0 + static_cast<double>(h));
+                for (uint64_t k = 0; k <= h && result == CRDFFT_OK; ++k)
                 {
-                    if (!checked(k, h + 1))
+                    const double re = X[k].real() - ((k == 1) ? static_cast<double>(h) : 0.0), im = X[k].imag();
+                    if (!(re * re + im * im <= limit * limit) && checked(k, h + 1)) // NaN as well
                     {
-                        continue;
+                        result = CRDFFT_SELF_CHECK_FAILED;
                     }
-                    const double want = (k == 1) ? static_cast<double>(h) : 0.0;
-                    const double err = std::abs(std::complex<double>(X[k].real() - want, X[k].imag()));
-                    if (!(err <= maxerr))
-                    {
-                        maxerr = err;
-                    }
-                }
-                if (!(maxerr <= tol * (1.0 + static_cast<double>(h))))
-                {
-                    result = CRDFFT_SELF_CHECK_FAILED;
                 }
             }
         }
@@ -334,23 +314,12 @@ extern "C" crdfft_status crdfft_self_check(crdfft_plan plan)
                 {
                     x[0] += 0.5f;
                 }
-                double maxerr = 0.0;
-                for (uint64_t j = 0; j < n; ++j)
+                for (uint64_t j = 0; j < n && result == CRDFFT_OK; ++j)
                 {
-                    if (!checked(j, n))
+                    if (!(std::abs(static_cast<double>(x[j]) - cosine[j]) <= tol * 2.0) && checked(j, n)) // NaN as well
                     {
-                        continue;
+                        result = CRDFFT_SELF_CHECK_FAILED;
                     }
-                    const double want = std::cos(kTwoPi * static_cast<double>(j) / static_cast<double>(n));
-                    const double err = std::abs(static_cast<double>(x[j]) - want);
-                    if (!(err <= maxerr))
-                    {
-                        maxerr = err;
-                    }
-                }
-                if (!(maxerr <= tol * 2.0))
-                {
-                    result = CRDFFT_SELF_CHECK_FAILED;
                 }
             }
         }
