@@ -325,20 +325,26 @@ def test_r2c_of_non_finite_rows(gpu, n, batch):
 
 
 def test_real_four_step_over_several_chunks(gpu, po):
-    """n = 2^16 real (half length 32768 on the four-step, 512 transforms per 128 MiB chunk in both directions) over
-    1030 rows: the fused row pass (R2C) and fused column pass (C2R) across two chunk boundaries and a partial last
-    chunk, checked on rows either side of each boundary."""
+    """n = 2^16 real (half length 32768 on the four-step, 512 transforms per 128 MiB chunk in both directions, as the
+    planner splits it; named, as a plan without tuning runs whole transforms) over 1030 rows: the fused row pass (R2C)
+    and fused column pass (C2R) across two chunk boundaries and a partial last chunk, checked on rows either side of
+    each boundary."""
     n, batch = 1 << 16, 1030
     h = n // 2
     x = po.normal_real(n * batch, 77).reshape(batch, n).astype(np.float32)
-    r2c = gpu.FftPlan(n, batch, "r2c")
-    c2r = gpu.FftPlan(n, batch, "c2r")
-    assert r2c.info()["algorithm"] == 2 and r2c.info()["chunk"] < batch
+    r2c = gpu.FftPlan(n, batch, "r2c", tuning={"chunk": 512})
+    c2r = gpu.FftPlan(n, batch, "c2r", tuning={"chunk": 512})
+    for plan, t in ((r2c, "r2c"), (c2r, "c2r")):
+        info = plan.info()
+        assert info["algorithm"] == 2 and info["whole"] == 0
+        assert {k: v for k, v in info.items() if k not in ("whole", "check", "table_bytes")} == {
+            k: v for k, v in gpu.describe(n, batch, t).items() if k not in ("whole", "check", "table_bytes")}
     xin = gpu.DeviceBuffer.from_array(x)
     spec = gpu.DeviceBuffer(8 * (h + 1) * batch)
     back = gpu.DeviceBuffer(4 * n * batch)
-    r2c.execute(xin, spec, gpu.FORWARD)
-    c2r.execute(spec, back, gpu.INVERSE)
+    for plan, src, dst, direction in ((r2c, xin, spec, gpu.FORWARD), (c2r, spec, back, gpu.INVERSE)):
+        acc = plan.execute_profiled(src, dst, direction)
+        assert [acc.launches[i] for i in range(4)] == [3, 3, 0, 0]  # both passes of 512, 512 and 6 rows
     gpu.synchronize()
     rows = [0, 1, 511, 512, 1022, 1023, 1024, 1025, batch - 1]
     X = spec.download((batch, h + 1), np.complex64)[rows]

@@ -122,6 +122,47 @@ def test_real_rounds_match_fp64_and_the_four_step(gpu, po, batch, pad):
             assert po.rel_l2(X[r, 1:h], Y[r, 1:h].astype(np.complex128)) <= 2 * bound(n), r
 
 
+# padded reals on both sides (even distances), padded bins, and bases at every residue of a 128-byte line: the R2C stores are laid
+# out by the residue of each row of bins, whichever of base and distance makes it
+@pytest.mark.parametrize("pad_real,pad_bins,base_real,base_bins", [(2, 0, 0, 0), (6, 3, 1, 1), (30, 15, 2, 5), (2, 14, 0, 8),
+                                                                   (10, 1, 3, 15), (0, 15, 7, 11), (64, 2, 16, 2)])
+def test_real_rows_at_any_distance_and_base(gpu, po, pad_real, pad_bins, base_real, base_bins):
+    """base_real pairs of reals and base_bins bins into their allocations; the gaps between rows keep what was there, and the
+    values equal those of packed rows bit for bit."""
+    n, batch = 1 << 16, 130
+    h = n // 2
+    ri, co = n + pad_real, h + 1 + pad_bins
+    print(f"whole real pads {pad_real} {pad_bins} bases {base_real} {base_bins}", flush=True)
+    rng = np.random.default_rng(pad_real + pad_bins)
+    x = rng.standard_normal((batch, n), dtype=np.float32)
+    packed = gpu.FftPlan(n, batch, "r2c")
+    spec, back = gpu.DeviceBuffer(8 * (h + 1) * batch), gpu.DeviceBuffer(4 * n * batch)
+    packed.execute(gpu.DeviceBuffer.from_array(x), spec, gpu.FORWARD)
+    gpu.FftPlan(n, batch, "c2r").execute(spec, back, gpu.INVERSE)
+    gpu.synchronize()
+    X, xb = spec.download((batch, h + 1), np.complex64), back.download((batch, n), np.float32)
+    rows = [0, 1, batch - 1]
+    assert po.rel_l2(X[rows], po.rfft64(x[rows].astype(np.float64))) <= bound(n)
+    reals = np.full(2 * base_real + batch * ri, -7.25, np.float32)
+    bins = np.full(base_bins + batch * co, np.complex64(complex(2.5, -1.5)))
+    reals[2 * base_real:].reshape(batch, ri)[:, :n] = x
+    src, dst = gpu.DeviceBuffer.from_array(reals), gpu.DeviceBuffer.from_array(bins)
+    r2c = gpu.FftPlan(n, batch, "r2c", idist=ri, odist=co)
+    c2r = gpu.FftPlan(n, batch, "c2r", idist=co, odist=ri)
+    assert r2c.info()["whole"] == c2r.info()["whole"] == batch
+    r2c.execute(src.address + 8 * base_real, dst.address + 8 * base_bins, gpu.FORWARD)
+    gpu.synchronize()
+    want = bins.copy()
+    want[base_bins:].reshape(batch, co)[:, : h + 1] = X
+    assert np.array_equal(dst.download(want.shape, np.complex64).view(np.uint32), want.view(np.uint32))
+    src.upload(np.full_like(reals, -7.25))
+    c2r.execute(dst.address + 8 * base_bins, src.address + 8 * base_real, gpu.INVERSE)
+    gpu.synchronize()
+    want = np.full_like(reals, -7.25)
+    want[2 * base_real:].reshape(batch, ri)[:, :n] = xb
+    assert np.array_equal(src.download(want.shape, np.float32).view(np.uint32), want.view(np.uint32))
+
+
 def test_rerun_of_the_real_forms_is_bit_identical(gpu):
     n, batch = 1 << 16, 300
     h = n // 2
