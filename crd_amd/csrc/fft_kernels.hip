@@ -888,12 +888,13 @@ __global__ __launch_bounds__(TH) void k_fused(FusedArgs a)
 // ---------------------------------------------------------------------------------------------------------------
 // The five passes of the chirp-z route (bluestein.hpp:82-135) with the m-point intermediate kept in registers and
 // LDS: the only HBM traffic is x in and X out (n points each) plus the L2-resident c and FFT_m(b) tables. The
-// zero padding and the k < n store guard are the buffer resources' range checks: reads at or past n return 0 and
-// writes there are dropped, as are all accesses of an inactive slot (num_records 0).
+// zero padding, the k < n store guard and inactive slots (no bytes) are range checks: reads at or past n return 0 and
+// writes there are dropped, by the buffer resource from 64 threads a sequence, below by a compare (Row<false, true>).
 // n <= N / 2, so the upper half of a thread's slots is padding on the way in and past the end on the way out: it is never
 // loaded, the first stage leaves out the butterflies that would add it (DftHalf), and the second transform's last stage
-// forms only the lower half (2^23 points: n = 127 67 -> 52 us, 1009 89 -> 76, 4001 113 -> 99). Bound by the vector unit and
-// LDS: two N-point transforms for n points, 4x the floor of its bytes at n = 1009. 16 values per thread: 1009 90 us.
+// forms only the lower half (2^23 points: n = 127 67 -> 52 us, 1009 89 -> 76, 4001 113 -> 99). Two N-point transforms for n
+// points: 3.4x the floor of its bytes at n = 1009 x 8192, where by counters LDS is busy 65 % of the time (half of that in bank
+// conflicts), the vector unit 58 %, and 7.4 waves a SIMD wait for one or the other. 16 values per thread: 1009 90 us.
 template <int N, int E, bool INV>
 __global__ __launch_bounds__((RowCfg<N, E>::threads)) void k_blue(BlueArgs a)
 {

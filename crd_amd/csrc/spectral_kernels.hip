@@ -75,8 +75,8 @@ __global__ __launch_bounds__((SpecCfg<H, E>::threads)) void k_spec(SpecArgs a)
     {
         const uint64_t f = group + it * groups;
         const bool active = f < a.frames;
-        // the tables are the same for every frame; an empty asm hides that from the frame loop, so the compiler reloads them per frame
-        // (L1/L2 hits) instead of holding every butterfly's twiddles in registers across the frame loop
+        // the tables are the same for every frame; an empty asm hides that from the frame loop, so the compiler reloads them
+        // per frame (L1/L2 hits) instead of holding every butterfly's twiddles in registers across the frame loop
         const cf* tw = reinterpret_cast<const cf*>(a.tw);
         const cf* wk = reinterpret_cast<const cf*>(a.wtab);
         const float* win = a.window;
@@ -84,8 +84,9 @@ __global__ __launch_bounds__((SpecCfg<H, E>::threads)) void k_spec(SpecArgs a)
         {
             asm volatile("" : "+s"(tw), "+s"(wk), "+s"(win));
         }
-        // the frame through a buffer resource: an inactive frame gets no records, so its loads read zeros and touch
-        // no memory
+        // From 64 threads a frame on a buffer resource: an inactive frame gets no records, so its loads read zeros and touch no
+        // memory. Below, plain loads: an inactive slot reads the first frame's samples. Its results go nowhere either way
+        // (`active` at every store and accumulation).
         const Row<(T >= 64)> xr(a.x + (active ? f * a.hop : 0), active ? 8u * H : 0u);
         cf v[E];
         if (pairs)
@@ -243,9 +244,11 @@ __global__ __launch_bounds__((SpecCfg<H, E>::threads)) void k_spec(SpecArgs a)
 // frame: a lane group of T = N/E threads adds |Z[k]|^2 of its pairs g, g + G, ... to its E slots, folds k onto
 // N - k through LDS once at the end and the workgroup writes one partial row of N/2 + 1 densities. Per frame that is half an N-point
 // transform (12 levels of 4096 points for two frames) in place of a half-length one, a recombine and its LDS exchange.
-// Bound by the vector unit (about 900 instructions a thread and pair at N = 4096, E = 16; floor by bytes 44 us). Measured,
-// 2^26 samples at 50 % overlap: N = 4096 268 -> 170 us, 1024 200 -> 112, 256 303 -> 97, 64 683 -> 88. Loading the next pair
-// ahead (32 more registers) measured no better, nor did reloading the twiddles per pair instead of keeping them.
+// Measured, 2^26 samples at 50 % overlap: N = 4096 257 -> 163 us, 1024 200 -> 111, 256 298 -> 90, 64 683 -> 88 (floor by bytes
+// 44). What bounds it at N = 4096, E = 16, by counters: the vector unit issues 56 % of the time, LDS is busy 32 % (9 % in bank
+// conflicts), and of the 3.3 waves a SIMD holds (LDS allows four) each spends a third of its time at waits and barriers and
+// another 43 % waiting to issue. Loading the next pair ahead (32 more registers) measured no better, nor did
+// reloading the twiddles per pair instead of keeping them.
 template <int N, int E> struct WelchCfg
 {
     static constexpr int T = N / E;

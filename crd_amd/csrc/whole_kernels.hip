@@ -366,20 +366,28 @@ template <int NT, bool INV, int KIND> __global__ __launch_bounds__(512) void k_w
     // C2R rows of h + 1 bins share lines with their neighbours: plain loads
     constexpr int kLoad = KIND == kWholeC2R ? 0 : kAuxNt;
 
-    // R2C: thread (w, b, i) and its 4 lower values k pair with the upper values, in reverse, of the thread that holds
-    // rows -k1: (7 - w, 3 - b, -i); half W_n^{256 k2} of its lower values
+    // R2C (NT = 4): output k = k1 + N1 k2. A set is 16 rows k1 (lanes i) of the lower half in waves 0..3 and their mirrors
+    // N1 - k1 in waves 4..7; of a thread's k2, the lower values low + 32 r (r < 4, kStep bins apart) stay and the upper ones
+    // low + 16 + 32 r are sent across.
+    constexpr int kVal = 4;                           // lower values a thread
+    constexpr int kCol = C::N2 / (2 * kVal);          // 16: k2 from a lower value to the upper one after it
+    constexpr uint32_t kStep = 2u * kCol * C::N1;     // 8192 bins between a thread's lower values
+    static_assert(NT != 4 || (kCol == 16 && kVal * kStep == C::N && C::threads == 512 && RM == 2),
+                  "the mirror rules below: 16 rows a set, 4 waves a half, 4 values a thread and half");
+    // thread (w, b, i) and its lower values k pair with the upper values, in reverse, of the thread that holds rows -k1:
+    // (7 - w, 3 - b, -i); half W_n^{N1 k2} of its lower values
     const int low = (w & 3) + 4 * b;
     const int cross = 64 * (7 - w) + 16 * (3 - b) + ((16 - i) & 15);
     // rows 0 and 128 (lanes i = 0 of the first set) are their own mirrors: k2 -> -k2 and 127 - k2
     const int cross0 = i != 0 ? cross
                               : (w < 4 ? 64 * ((16 - low) & 3) + 16 * (((16 - low) >> 2) & 3) : 64 * (11 - w) + 16 * (3 - b));
-    cf wk2[4];
+    cf wk2[kVal];
     if constexpr (KIND == kWholeR2C)
     {
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
+        for (int r = 0; r < kVal; ++r)
         {
-            const cf x = reinterpret_cast<const cf*>(a.roots)[low + 32 * r];
+            const cf x = reinterpret_cast<const cf*>(a.roots)[low + 2 * kCol * r];
             wk2[r] = cf{0.5f * x.x, 0.5f * x.y};
         }
     }
@@ -677,7 +685,7 @@ template <int NT, bool INV, int KIND> __global__ __launch_bounds__(512) void k_w
         // from a set's address back to the one before: rows 16 lower (w < 4) or higher
         const uint32_t back = now ? 0u : (w < 4 ? 0u - 128u : 128u);
         const uint32_t back_h = now_h ? 0u : (w < 4 ? 128u : 0u - 128u);
-        const bool odd_row = i == 0 && w >= 4; // row 128 in the first set, not row 256
+        const bool odd_row = i == 0 && w >= 4; // row N1 / 2 in the first set, not row N1
         constexpr uint32_t kFar = 0x40000000u; // outside the resource: dropped
         cf old[4], old_h[4];
         auto cross_store = [&](int j) {
@@ -685,10 +693,13 @@ template <int NT, bool INV, int KIND> __global__ __launch_bounds__(512) void k_w
             // through an empty asm, so that the addresses of all sets are not kept in registers across transforms
             int iv = i, lowv = low;
             asm volatile("" : "+v"(iv), "+v"(lowv));
-            const int k1 = w < 4 ? iv + 16 * j : iv + 240 - 16 * j + (iv == 0 ? (j == 0 ? -112 : 16) : 0);
+            // lower waves: rows i + 16 j; upper waves: rows i + N1 - 16 (j + 1), but for i = 0, whose lower row 16 j mirrors to
+            // N1 - 16 j, one set on (row N1 / 2 in the first set: rows 0 and N1 / 2 are their own mirrors)
+            constexpr int kTop = C::N1 - 16;
+            const int k1 = w < 4 ? iv + 16 * j : iv + kTop - 16 * j + (iv == 0 ? (j == 0 ? C::N1 / 2 - kTop : 16) : 0);
             const cf wk = wk1[k1];
-            const uint32_t k = static_cast<uint32_t>(k1 + 256 * lowv); // k + 8192 r, r < 4
-            uint32_t at = k * 8u, at_h = (C::N - k - 3u * 8192u) * 8u;
+            const uint32_t k = static_cast<uint32_t>(k1 + C::N1 * lowv); // k + kStep r
+            uint32_t at = k * 8u, at_h = (C::N - k - (kVal - 1) * kStep) * 8u;
             cf p[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r)
@@ -697,8 +708,9 @@ template <int NT, bool INV, int KIND> __global__ __launch_bounds__(512) void k_w
             }
             if (j == 0)
             {
-                // in thread 0 k = 8192 r mirrors within the thread, and so do its upper values k = 4096 + 8192 r (the
-                // other threads' stores of those are dropped)
+                // in thread 0 k = kStep r mirrors within the thread, and so do its upper values k = kMid + kStep r (the other
+                // threads' stores of those are dropped)
+                constexpr uint32_t kMid = static_cast<uint32_t>(kCol * C::N1), kMid1 = kMid + kStep;
                 const bool t0 = tid == 0;
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
@@ -708,12 +720,12 @@ template <int NT, bool INV, int KIND> __global__ __launch_bounds__(512) void k_w
                 }
                 const uint32_t far = t0 ? 0u : kFar;
                 cf xk, xh;
-                mirror_pair(x[0], x[3 * 512], cf{0.5f * W<16, 256>::re, 0.5f * W<16, 256>::im}, xk, xh);
-                bst<0>(dst, far, 4096u * 8u, xk);
-                bst<0>(dst, far, (C::N - 4096u) * 8u, xh);
-                mirror_pair(x[512], x[2 * 512], cf{0.5f * W<48, 256>::re, 0.5f * W<48, 256>::im}, xk, xh);
-                bst<0>(dst, far, 12288u * 8u, xk);
-                bst<0>(dst, far, (C::N - 12288u) * 8u, xh);
+                mirror_pair(x[0], x[3 * 512], cf{0.5f * W<kCol, C::N1>::re, 0.5f * W<kCol, C::N1>::im}, xk, xh);
+                bst<0>(dst, far, kMid * 8u, xk);
+                bst<0>(dst, far, (C::N - kMid) * 8u, xh);
+                mirror_pair(x[512], x[2 * 512], cf{0.5f * W<3 * kCol, C::N1>::re, 0.5f * W<3 * kCol, C::N1>::im}, xk, xh);
+                bst<0>(dst, far, kMid1 * 8u, xk);
+                bst<0>(dst, far, (C::N - kMid1) * 8u, xh);
                 at = now || odd_row ? at : kFar;
                 at_h = now_h || odd_row ? at_h : kFar;
             }
@@ -733,7 +745,7 @@ template <int NT, bool INV, int KIND> __global__ __launch_bounds__(512) void k_w
                     xk = tid == 0 ? cf{z[0].x + z[0].y, 0.0f} : xk;
                     xh = tid == 0 ? cf{z[0].x - z[0].y, 0.0f} : xh;
                 }
-                const uint32_t step = 65536u * static_cast<uint32_t>(r), step_h = 65536u * static_cast<uint32_t>(3 - r);
+                const uint32_t step = kStep * 8u * static_cast<uint32_t>(r), step_h = kStep * 8u * static_cast<uint32_t>(kVal - 1 - r);
                 if (j == 0)
                 {
                     bst<0>(dst, at, step, xk);
@@ -751,12 +763,12 @@ template <int NT, bool INV, int KIND> __global__ __launch_bounds__(512) void k_w
             {
                 // what the last set left for a line that no set follows
                 at = now ? kFar : k * 8u;
-                at_h = now_h ? kFar : (C::N - k - 3u * 8192u) * 8u;
+                at_h = now_h ? kFar : (C::N - k - (kVal - 1) * kStep) * 8u;
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
                 {
-                    bst<0>(dst, at, 65536u * static_cast<uint32_t>(r), old[r]);
-                    bst<0>(dst, at_h, 65536u * static_cast<uint32_t>(3 - r), old_h[r]);
+                    bst<0>(dst, at, kStep * 8u * static_cast<uint32_t>(r), old[r]);
+                    bst<0>(dst, at_h, kStep * 8u * static_cast<uint32_t>(kVal - 1 - r), old_h[r]);
                 }
             }
         };
