@@ -536,7 +536,7 @@ def main():
         head = xout.download((4096,), np.complex64)  # the first 32 KiB of the output of the last execute
         per_shape.append({"n": n, "batch": batch, "ms": round(ms, 4), "gbs": round(gbs, 1),
                           "ffts_per_s": round(batch / (ms * 1e-3), 1), "plan": {k: info[k] for k in (
-                              "algorithm", "n1", "n2", "e", "e1", "tile1", "e2", "tile2", "chunk")},
+                              "algorithm", "n1", "n2", "e", "e1", "tile1", "e2", "tile2", "chunk", "whole")},
                           "kernels": kernels, "transform_level": kernels_transform,
                           "output_head_fnv1a64": fnv1a64(head.tobytes())})
     result["per_shape"] = per_shape
